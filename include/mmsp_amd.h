@@ -275,12 +275,17 @@ int mmspx_set_tile(mmspx_state* s, int ty, int tz, int chunk);
  * the FP64 form with 8 fields on 8 x 32 only; an odd last step runs body 8)
  * and, for Ostwald ripening (2, 3 or 4 fields, 8 x 64 and 16 x 32 tiles),
  * its two passes in one march with w kept in LDS; the tile follows the body
- * (16 x 32 where the current tile is not one of those). */
+ * (16 x 32 where the current tile is not one of those). 2-D Allen-Cahn and
+ * Cahn-Hilliard (deterministic chemical potentials) in the MMSPX_F64 and
+ * MMSPX_F32 forms, each axis periodic on both sides or on neither: 13 and 14
+ * are the multi-step wave strips, 1 x 48 and 1 x 56 tiles of `chunk` rows,
+ * which take 8 and 4 Allen-Cahn or 4 and 2 Cahn-Hilliard steps per pass in
+ * registers (their default). */
 int mmspx_set_tile_options(mmspx_state* s, int body);
 /* Returns variant + 16 * tile body (1: register queues, or the 2-D
  * grain-growth tile; 2: wave strips, or 3-D register queues on 768 threads;
  * 3: temporal blocks, or 3-D register queues on 1024 threads; 4 and 5: the
- * split strips on two and four waves). Before any tile is set, reports what the last step ran
+ * split strips on two and four waves; 13 and 14: the multi-step wave strips). Before any tile is set, reports what the last step ran
  * (the Cahn-Hilliard default before any step). */
 int mmspx_get_tile(const mmspx_state* s, int* ty, int* tz, int* chunk);
 /* Project autotuner: times every candidate tile for `model` on this state's

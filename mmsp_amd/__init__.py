@@ -322,7 +322,9 @@ class Grid:
         and grain growth on 1 x 64 strips: 2 wave strips; 4 and 5 the split
         strips, 9, 10 and 11 the split strips two steps per pass (2-D
         periodic); 8 the 3-D plane march; 12 the 3-D plane march two steps per
-        pass (periodic; Ostwald ripening: its two passes in one march)."""
+        pass (periodic; Ostwald ripening: its two passes in one march); 13 and
+        14 the 2-D multi-step wave strips of Allen-Cahn and Cahn-Hilliard
+        (eight or four levels of the update per pass)."""
         check(lib.mmspx_set_tile_options(self._h, int(body) if body is not None else (1 if register_queues else 0)))
 
     def get_tile(self):

@@ -462,9 +462,12 @@ int mmspx_set_tile(mmspx_state* s, int ty, int tz, int chunk)
 	                        (s->tile.opt >= 4 && s->geom.dim == 2)))
 	              ? s->tile.opt
 	              : 0;
+	if (opt >= 13) opt = 0;
 	if (s->geom.dim == 2 && ty > 1 && tz == kTbCols) opt = 3;
 	else if (s->geom.dim == 2 && ty > 1) opt = 1;
 	else if (s->geom.dim == 2 && s->tuned && s->tile.ty > 1) opt = 0;
+	// 1 x 48 and 1 x 56 name the 2-D multi-step wave strips
+	if (s->geom.dim == 2 && ty == 1 && (tz == kSteps8Cols || tz == kSteps4Cols)) opt = tz == kSteps8Cols ? 13 : 14;
 	// 3-D two-step bodies: 32 x 32 tiles run body 7 only; body 6 runs 32 x 64
 	if (s->geom.dim == 3 && ty == 32 && tz == 32) opt = 7;
 	else if (s->geom.dim == 3 && s->tuned && s->tile.opt == 6 && ty == 32 && tz == 64) opt = 6;
@@ -479,19 +482,22 @@ int mmspx_set_tile(mmspx_state* s, int ty, int tz, int chunk)
 int mmspx_set_tile_options(mmspx_state* s, int body)
 {
 	if (!s) return fail(MMSPX_EINVAL, "null state");
-	if (body < 0 || body > 12 || (body == 3 && s->geom.dim != 3) ||
-	    ((body == 4 || body == 5 || (body >= 9 && body <= 11)) && s->geom.dim != 2) ||
+	if (body < 0 || body > 14 || (body == 3 && s->geom.dim != 3) ||
+	    ((body == 4 || body == 5 || (body >= 9 && body <= 11) || body >= 13) && s->geom.dim != 2) ||
 	    (((body >= 6 && body <= 8) || body == 12) && s->geom.dim != 3))
 		return fail(MMSPX_EINVAL, "unknown tile body");
 	if (!s->tuned) {
-		s->tile = default_choice(s->geom, s->desc.precision, MMSPX_CH_DW);
+		s->tile = one_step_choice(s->geom, s->desc.precision, MMSPX_CH_DW);
 		s->tuned = true;
 	}
 	s->tile.opt = body;
 	// 2-D: the split strips run 1 x 64 strips (bodies 4, 5), two steps per
 	// pass 1 x kChWaveOut (bodies 9, 10)
 	if (s->geom.dim == 2 && s->tile.variant == 2) {
-		if (body >= 9 && body <= 11) {
+		if (body >= 13) {
+			s->tile.ty = 1;
+			s->tile.tz = body == 13 ? kSteps8Cols : kSteps4Cols;
+		} else if (body >= 9 && body <= 11) {
 			s->tile.ty = 1;
 			s->tile.tz = kChWaveOut;
 		} else if (body == 4 || body == 5) {

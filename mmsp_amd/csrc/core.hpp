@@ -132,6 +132,9 @@ constexpr int kChWaveOut = 60;
 // one pass takes (tile plus halo fits the 64 lanes of a wave)
 constexpr int kTbCols = 48;
 constexpr int kTbMaxSteps = 8;
+// output columns of the multi-step wave strips: eight or four levels' halo each side
+constexpr int kSteps8Cols = 48;
+constexpr int kSteps4Cols = 56;
 
 // ---- kernel launchers (kernels_generic.hip, kernels_fused.hip, reduce.hip) ----
 // Each returns 0 or a negative code; all enqueue on `st`.
@@ -148,6 +151,8 @@ int launch_fused_step(const Geom& g, int prec, const ModelParams& p, const void*
 bool fused_needs_plane(const Geom& g, int model, const TuneChoice& t);
 int fused_steps_per_launch(int model, const TuneChoice& t);
 TuneChoice default_choice(const Geom& g, int prec, int model);
+// the default without the 2-D multi-step wave strips
+TuneChoice one_step_choice(const Geom& g, int prec, int model);
 int launch_reduce(const Geom& g, int prec, int what, const ModelParams& p, const void* a, double* part,
                   hipStream_t st);
 int launch_transpose(const void* src, void* dst, int nodes, int fields, size_t elem, bool to_field_major,
@@ -155,6 +160,14 @@ int launch_transpose(const void* src, void* dst, int nodes, int fields, size_t e
 int launch_convert(const void* src, int src_f64, void* dst, int dst_f64, int64_t n, hipStream_t st);
 int launch_copy(const void* src, void* dst, size_t bytes, hipStream_t st);
 bool tile_known(const Geom& g, const TuneChoice& t);
+// 2-D multi-step wave strips (kernels_steps2d.hip): tile bodies 13 (strips of
+// 48 columns) and 14 (56), `chunk` rows per wave; a pass takes up to
+// steps2d_max_steps steps
+bool steps2d_supported(const Geom& g, int prec, int model);
+int steps2d_max_steps(int model, int body);
+bool steps2d_choice(const Geom& g, int prec, int model, TuneChoice* out);
+int launch_steps2d(const Geom& g, int prec, const ModelParams& p, const void* a, void* b, hipStream_t st, int body,
+                   int chunk, int nsteps);
 int tile_candidates(const Geom& g, int prec, int model, TuneChoice* out, int max);
 
 // host-side compensated sum of the (sum, comp) partial pairs

@@ -412,9 +412,16 @@ static bool march2_choice(const Geom& g, int prec, int model, TuneChoice* out)
 	return true;
 }
 
+TuneChoice default_choice(const Geom& g, int prec, int model)
+{
+	TuneChoice t;
+	if (steps2d_choice(g, prec, model, &t)) return t;
+	return one_step_choice(g, prec, model);
+}
+
 // Defaults come from sweeps of the candidates below on MI355X (the figures
 // quoted are microseconds per step from those sweeps).
-TuneChoice default_choice(const Geom& g, int prec, int model)
+TuneChoice one_step_choice(const Geom& g, int prec, int model)
 {
 	if (!fused_supported(g, prec, model)) return TuneChoice{1, 0, 0, 0, 0};
 	const int64_t nodes = g.nodes;
@@ -580,6 +587,8 @@ bool tile_known(const Geom& g, const TuneChoice& t)
 		return (t.ty == 8 && t.tz == 64) || (t.ty == 16 && t.tz == 64) || (t.ty == 32 && t.tz == 64) ||
 		       (t.ty == 8 && t.tz == 32) || (t.ty == 4 && t.tz == 128) || (t.ty == 32 && t.tz == 32) ||
 		       (t.ty == 16 && t.tz == 32);
+	if (g.dim == 2 && (t.opt == 13 || t.opt == 14))
+		return t.ty == 1 && t.tz == (t.opt == 13 ? kSteps8Cols : kSteps4Cols);
 	if (g.dim == 2)
 		return (t.ty == 1 && (t.tz == 64 || t.tz == 128 || t.tz == 256 || t.tz == kChWaveOut)) ||
 		       ((t.ty == 8 || t.ty == 16 || t.ty == 32) && t.tz == kTbCols && t.chunk <= kTbMaxSteps) ||
@@ -690,6 +699,12 @@ int tile_candidates(const Geom& g, int prec, int model, TuneChoice* out, int max
 		if ((model == MMSPX_GG || model == MMSPX_ZENER) && (g.fields == 2 || g.fields == 4 || g.fields == 8) &&
 		    all_periodic(g))
 			for (int c : {8, 16, 32, 64}) add(1, kChWaveOut, c, 11);
+		// Allen-Cahn and Cahn-Hilliard: several steps per pass in registers
+		if (steps2d_supported(g, prec, model))
+			for (int c : {4, 8, 16, 32, 64}) {
+				add(1, kSteps8Cols, c, 13);
+				add(1, kSteps4Cols, c, 14);
+			}
 		// periodic Allen-Cahn: temporal blocks (chunk = steps per pass)
 		if (model == MMSPX_AC && all_periodic(g))
 			for (int tx : {8, 16, 32})
@@ -1282,6 +1297,7 @@ static int launch_prec(const Geom& g, const ModelParams& p, const void* a, void*
                        int nsteps, void* aux)
 {
 	const int chunk = t.chunk > 0 ? t.chunk : 32;
+	if (g.dim == 2 && (t.opt == 13 || t.opt == 14)) return launch_steps2d(g, PREC, p, a, b, st, t.opt, chunk, nsteps);
 	switch (p.model) {
 	case MMSPX_CH: return launch_ch_prec<PREC, 0>(g, p, a, b, st, t, nsteps);
 	case MMSPX_CH_DW: return launch_ch_prec<PREC, 1>(g, p, a, b, st, t, nsteps);
@@ -1355,6 +1371,8 @@ bool fused_needs_plane(const Geom& g, int model, const TuneChoice& t)
 
 int fused_steps_per_launch(int model, const TuneChoice& t)
 {
+	if ((model == MMSPX_AC || model == MMSPX_CH || model == MMSPX_CH_DW) && (t.opt == 13 || t.opt == 14))
+		return steps2d_max_steps(model, t.opt);
 	if (model == MMSPX_AC && t.tz == kTbCols) return std::max(1, std::min(t.chunk, kTbMaxSteps));
 	if ((model == MMSPX_CH || model == MMSPX_CH_DW) && (t.opt == 6 || t.opt == 7)) return 2;
 	if ((model == MMSPX_GG || model == MMSPX_ZENER) && t.opt >= 9 && t.opt <= 11) return 2;
