@@ -280,7 +280,12 @@ int mmspx_set_tile(mmspx_state* s, int ty, int tz, int chunk);
  * MMSPX_F32 forms, each axis periodic on both sides or on neither: 13 and 14
  * are the multi-step wave strips, 1 x 48 and 1 x 56 tiles of `chunk` rows,
  * which take 8 and 4 Allen-Cahn or 4 and 2 Cahn-Hilliard steps per pass in
- * registers (their default). */
+ * registers (their default). 3-D periodic Allen-Cahn and Cahn-Hilliard
+ * (deterministic chemical potentials) in the same forms: 15 is the four-level
+ * march, four Allen-Cahn or two Cahn-Hilliard steps per pass on 26 x 52, 32 x
+ * 32, 16 x 32 and 16 x 16 tiles, in the FP64 form also 16 x 64, in FP32 32 x 64
+ * (their default where it is the fastest; a default reports the body of the
+ * pass it stands for, 7 for Cahn-Hilliard and 12 or 8 for Allen-Cahn). */
 int mmspx_set_tile_options(mmspx_state* s, int body);
 /* Returns variant + 16 * tile body (1: register queues, or the 2-D
  * grain-growth tile; 2: wave strips, or 3-D register queues on 768 threads;

@@ -324,7 +324,8 @@ class Grid:
         periodic); 8 the 3-D plane march; 12 the 3-D plane march two steps per
         pass (periodic; Ostwald ripening: its two passes in one march); 13 and
         14 the 2-D multi-step wave strips of Allen-Cahn and Cahn-Hilliard
-        (eight or four levels of the update per pass)."""
+        (eight or four levels of the update per pass); 15 their 3-D four-level
+        march (periodic)."""
         check(lib.mmspx_set_tile_options(self._h, int(body) if body is not None else (1 if register_queues else 0)))
 
     def get_tile(self):

@@ -377,6 +377,7 @@ static int step_impl(mmspx_state* s, int model, const double* params, int np, in
 		return fail(MMSPX_EUNSUPPORTED, "no tiled/fused kernel for this model, shape and boundary condition");
 	}
 	s->last = fused ? tc : TuneChoice{1, 0, 0, 0, 0};
+	if (s->last.opt == 15) s->last.opt = march4_reported_body(g, model);
 	s->has_last = true;
 	const int spl = fused ? fused_steps_per_launch(model, tc) : 1;
 	if ((((ch_family(model) || model == MMSPX_OSTWALD) && !fused) || (fused && fused_needs_plane(g, model, tc))) &&
@@ -472,6 +473,10 @@ int mmspx_set_tile(mmspx_state* s, int ty, int tz, int chunk)
 	if (s->geom.dim == 3 && ty == 32 && tz == 32) opt = 7;
 	else if (s->geom.dim == 3 && s->tuned && s->tile.opt == 6 && ty == 32 && tz == 64) opt = 6;
 	else if (s->geom.dim == 3 && s->tuned && (s->tile.opt == 8 || s->tile.opt == 12)) opt = s->tile.opt;
+	// 26 x 52 and 16 x 16 name the 3-D four-level march
+	if (s->geom.dim == 3 && ((s->tuned && s->tile.opt == 15 && march4_tile_known(s->desc.precision, ty, tz)) ||
+	                         (ty == 26 && tz == 52) || (ty == 16 && tz == 16)))
+		opt = 15;
 	TuneChoice t{2, ty, tz, chunk, opt};
 	if (!tile_known(s->geom, t)) return fail(MMSPX_EINVAL, "no compiled tile of that shape for this grid");
 	s->tile = t;
@@ -482,9 +487,10 @@ int mmspx_set_tile(mmspx_state* s, int ty, int tz, int chunk)
 int mmspx_set_tile_options(mmspx_state* s, int body)
 {
 	if (!s) return fail(MMSPX_EINVAL, "null state");
-	if (body < 0 || body > 14 || (body == 3 && s->geom.dim != 3) ||
-	    ((body == 4 || body == 5 || (body >= 9 && body <= 11) || body >= 13) && s->geom.dim != 2) ||
-	    (((body >= 6 && body <= 8) || body == 12) && s->geom.dim != 3))
+	if (body < 0 || body > 15 || (body == 3 && s->geom.dim != 3) ||
+	    ((body == 4 || body == 5 || (body >= 9 && body <= 11) || body == 13 || body == 14) &&
+	     s->geom.dim != 2) ||
+	    (((body >= 6 && body <= 8) || body == 12 || body == 15) && s->geom.dim != 3))
 		return fail(MMSPX_EINVAL, "unknown tile body");
 	if (!s->tuned) {
 		s->tile = one_step_choice(s->geom, s->desc.precision, MMSPX_CH_DW);
@@ -510,7 +516,12 @@ int mmspx_set_tile_options(mmspx_state* s, int body)
 	// two-step march 16 x 32 for every model)
 	if (s->geom.dim == 3 && s->tile.variant == 2) {
 		const int ty = s->tile.ty, tz = s->tile.tz;
-		if (body == 12) {
+		if (body == 15) {
+			if (!march4_tile_known(s->desc.precision, ty, tz)) {
+				s->tile.ty = 16;
+				s->tile.tz = 32;
+			}
+		} else if (body == 12) {
 			if (!((ty == 16 && tz == 32) || (ty == 16 && tz == 64) || (ty == 32 && tz == 64) || (ty == 8 && tz == 64) ||
 			      (ty == 8 && tz == 32))) {
 				s->tile.ty = 16;
@@ -536,6 +547,7 @@ int mmspx_get_tile(const mmspx_state* s, int* ty, int* tz, int* chunk)
 {
 	if (!s) return fail(MMSPX_EINVAL, "null state");
 	TuneChoice t = s->tuned ? s->tile : s->has_last ? s->last : default_choice(s->geom, s->desc.precision, MMSPX_CH_DW);
+	if (!s->tuned && t.opt == 15) t.opt = march4_reported_body(s->geom, MMSPX_CH_DW);
 	if (ty) *ty = t.ty;
 	if (tz) *tz = t.tz;
 	if (chunk) *chunk = t.chunk;
@@ -598,8 +610,8 @@ int mmspx_autotune(mmspx_state* s, int model, const double* params, int np, int 
 	int rc = make_params(model, params, np, &p);
 	if (rc) return rc;
 	std::string rep;
-	TuneChoice cand[64];
-	int nc = fused_supported(s->geom, s->desc.precision, model) ? tile_candidates(s->geom, s->desc.precision, model, cand, 64) : 0;
+	TuneChoice cand[96];
+	int nc = fused_supported(s->geom, s->desc.precision, model) ? tile_candidates(s->geom, s->desc.precision, model, cand, 96) : 0;
 	// keep the state: every trial starts from it and it is restored at the end
 	void* saved = nullptr;
 	if (hipMalloc(&saved, s->bytes) != hipSuccess) return fail(MMSPX_ENOMEM, "device allocation failed");

@@ -151,7 +151,7 @@ int launch_fused_step(const Geom& g, int prec, const ModelParams& p, const void*
 bool fused_needs_plane(const Geom& g, int model, const TuneChoice& t);
 int fused_steps_per_launch(int model, const TuneChoice& t);
 TuneChoice default_choice(const Geom& g, int prec, int model);
-// the default without the 2-D multi-step wave strips
+// the default without the 2-D multi-step wave strips and the four-level march
 TuneChoice one_step_choice(const Geom& g, int prec, int model);
 int launch_reduce(const Geom& g, int prec, int what, const ModelParams& p, const void* a, double* part,
                   hipStream_t st);
@@ -160,6 +160,15 @@ int launch_transpose(const void* src, void* dst, int nodes, int fields, size_t e
 int launch_convert(const void* src, int src_f64, void* dst, int dst_f64, int64_t n, hipStream_t st);
 int launch_copy(const void* src, void* dst, size_t bytes, hipStream_t st);
 bool tile_known(const Geom& g, const TuneChoice& t);
+// 3-D four-level march (kernels_march4.hip), tile body 15: two Cahn-Hilliard
+// or four Allen-Cahn steps per pass on periodic grids
+bool march4_supported(const Geom& g, int prec, int model);
+int march4_max_steps(int model);
+bool march4_tile_known(int prec, int ty, int tz);
+bool march4_choice(const Geom& g, int prec, int model, TuneChoice* out);
+int march4_reported_body(const Geom& g, int model);
+int launch_march4(const Geom& g, int prec, const ModelParams& p, const void* a, void* b, hipStream_t st,
+                  const TuneChoice& t, int nsteps);
 // 2-D multi-step wave strips (kernels_steps2d.hip): tile bodies 13 (strips of
 // 48 columns) and 14 (56), `chunk` rows per wave; a pass takes up to
 // steps2d_max_steps steps

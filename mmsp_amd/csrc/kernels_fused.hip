@@ -353,55 +353,25 @@ static TuneChoice two_step_choice(const Geom& g, int prec)
 	return best;
 }
 
-// Periodic 3-D Allen-Cahn, grain growth and Zener pinning: the plane march
-// two steps per pass (body 12) where its 64-node tile rows fit the last axis
-// (padding at most an eighth of it: 160^3 Allen-Cahn FP64 pads to 192 and
-// takes 15.5 us per step against 14.1 for the one-step march).
-// Allen-Cahn: 16 x 64 or 32 x 64 tiles and the chunk from the cost model of
-// two_step_choice: rounds x (chunk + 3 planes: the halo plane on each side
-// and the queue's first load) x owned points per thread (16 x 64: 1188 on
-// 640 threads, two workgroups per CU in rounds of 512 each 1.7 times as
-// long; 32 x 64: 2244 on 768, one per CU). It picks the measured best, or
-// one within 5 %, at every side swept (us per step, against the one-step
-// march): FP64 64^3 16 x 64 with 4-plane chunks 4.3 (5.7), 128^3 16 x 64
-// with 8 7.2 (10.3), 192^3 32 x 64 with 16 16.7 (21.9), 256^3 32 x 64 with
-// 32 30.0 (43.9; 16 x 64 29.8); FP32 64^3 3.6 (6.9), 128^3 5.6 (8.0; 32 x 64
-// with 4: 5.3), 192^3 11.2 (15.7), 256^3 19.0 (24.3).
-// Grain growth and Zener pinning (2 or 4 fields; 8 in FP32 from 2^22 nodes):
-// 8 x 64 tiles (one node and its halo per thread, 704 threads), 64-plane
-// chunks halved until a launch has 256 workgroups per CU that fit (two for
-// 2 fields, one otherwise by registers): 256^3 x 2 FP64 81.0 (117.0), x 4
-// FP64 178.6 (239.6), x 4 FP32 111.8 (125.2), x 8 FP32 222.0 (253.3); Zener
-// x 2 FP32 34.7 (54.8), x 4 107.0 (122.4); 192^3 x 8 FP32 109.1 (125.6);
-// 128^3 x 2 FP32 8.6 (12.2), x 4 FP64 24.6 (27.4); 64^3 x 4 FP32 5.6 (7.1).
-// 128^3 x 8 FP32 gains nothing (29.5 against 28.6), and 8 FP64 fields fit
-// the LDS on 8 x 32 tiles only (256^3: 488.5 against 481.0): those stay on
-// the one-step march.
+// Periodic 3-D grain growth and Zener pinning (2 or 4 fields; 8 in FP32 from
+// 2^22 nodes): the plane march two steps per pass (body 12) where its 64-node
+// tile rows fit the last axis (padding at most an eighth of it): 8 x 64 tiles
+// (one node and its halo per thread, 704 threads), 64-plane chunks halved
+// until a launch has 256 workgroups per CU that fit (two for 2 fields, one
+// otherwise by registers): 256^3 x 2 FP64 81.0 us per step against 117.0 for
+// the one-step march, x 4 FP64 178.6 (239.6), x 4 FP32 111.8 (125.2), x 8 FP32
+// 222.0 (253.3); Zener x 2 FP32 34.7 (54.8), x 4 107.0 (122.4); 192^3 x 8 FP32
+// 109.1 (125.6); 128^3 x 2 FP32 8.6 (12.2), x 4 FP64 24.6 (27.4); 64^3 x 4
+// FP32 5.6 (7.1). 128^3 x 8 FP32 gains nothing (29.5 against 28.6), and 8 FP64
+// fields fit the LDS on 8 x 32 tiles only (256^3: 488.5 against 481.0): those
+// stay on the one-step march.
 static bool march2_choice(const Geom& g, int prec, int model, TuneChoice* out)
 {
 	constexpr int kCUs = 256;
 	if (!all_periodic(g) || (prec != MMSPX_F64 && prec != MMSPX_F32)) return false;
-	if (model != MMSPX_AC && model != MMSPX_GG && model != MMSPX_ZENER) return false;
+	if (model != MMSPX_GG && model != MMSPX_ZENER) return false;
 	const int nz = g.n[2], pad = (nz + 63) / 64 * 64 - nz;
 	if (pad * 8 > nz) return false;
-	if (model == MMSPX_AC) {
-		double best_cost = 1e300;
-		for (int ty : {16, 32}) {
-			const double own = ty == 16 ? 1188.0 / 640 : 2244.0 / 768;
-			const int64_t tiles = (int64_t)((g.n[1] + ty - 1) / ty) * ((nz + 63) / 64);
-			for (int c : {4, 8, 16, 32, 64}) {
-				const int64_t wgs = tiles * ((g.n[0] + c - 1) / c);
-				const double rounds = (ty == 16 && wgs > kCUs) ? 1.7 * (double)((wgs + 2 * kCUs - 1) / (2 * kCUs))
-				                                               : (double)((wgs + kCUs - 1) / kCUs);
-				const double cost = rounds * (c + 3) * own;
-				if (cost < best_cost) {
-					best_cost = cost;
-					*out = TuneChoice{2, ty, 64, c, 12};
-				}
-			}
-		}
-		return true;
-	}
 	const int q = g.fields;
 	if (!(q == 2 || q == 4 || (q == 8 && prec == MMSPX_F32 && g.nodes >= ((int64_t)1 << 22)))) return false;
 	const int per_cu = q == 2 ? 2 : 1;
@@ -416,6 +386,7 @@ TuneChoice default_choice(const Geom& g, int prec, int model)
 {
 	TuneChoice t;
 	if (steps2d_choice(g, prec, model, &t)) return t;
+	if (march4_choice(g, prec, model, &t)) return t;
 	return one_step_choice(g, prec, model);
 }
 
@@ -583,6 +554,8 @@ TuneChoice one_step_choice(const Geom& g, int prec, int model)
 bool tile_known(const Geom& g, const TuneChoice& t)
 {
 	if (t.chunk < 2 || t.chunk > 4096) return false;
+	if (g.dim == 3 && t.opt == 15)
+		return march4_tile_known(MMSPX_F64, t.ty, t.tz) || march4_tile_known(MMSPX_F32, t.ty, t.tz);
 	if (g.dim == 3)
 		return (t.ty == 8 && t.tz == 64) || (t.ty == 16 && t.tz == 64) || (t.ty == 32 && t.tz == 64) ||
 		       (t.ty == 8 && t.tz == 32) || (t.ty == 4 && t.tz == 128) || (t.ty == 32 && t.tz == 32) ||
@@ -641,6 +614,9 @@ int tile_candidates(const Geom& g, int prec, int model, TuneChoice* out, int max
 		// (Ostwald ripening: the one-pass march)
 		const bool two = all_periodic(g) && model != MMSPX_AC_NOISE && model != MMSPX_GG_ANISO &&
 		                 (prec == MMSPX_F64 || prec == MMSPX_F32);
+		if (march4_supported(g, prec, model))
+			for (int c : {4, 8, 16, 32, 64})
+				for (auto& t : {std::pair<int, int>{26, 52}, {32, 32}, {16, 32}, {16, 16}}) add(t.first, t.second, c, 15);
 		if (two)
 			for (int c : {8, 16, 32, 64}) {
 				if (scalar) {
@@ -669,6 +645,10 @@ int tile_candidates(const Geom& g, int prec, int model, TuneChoice* out, int max
 		// two steps per pass (deterministic chemical potentials, periodic grids)
 		if ((model == MMSPX_CH || model == MMSPX_CH_DW) && !edges)
 			for (int c : {6, 8, 12, 16, 24, 32, 48, 64}) {
+				if (march4_supported(g, prec, model) && c != 6 && c != 12) {
+					add(26, 52, c, 15);
+					add(16, 32, c, 15);
+				}
 				add(32, 64, c, 6);
 				add(32, 32, c, 7);
 			}
@@ -1298,6 +1278,7 @@ static int launch_prec(const Geom& g, const ModelParams& p, const void* a, void*
 {
 	const int chunk = t.chunk > 0 ? t.chunk : 32;
 	if (g.dim == 2 && (t.opt == 13 || t.opt == 14)) return launch_steps2d(g, PREC, p, a, b, st, t.opt, chunk, nsteps);
+	if (g.dim == 3 && t.opt == 15) return launch_march4(g, PREC, p, a, b, st, t, nsteps);
 	switch (p.model) {
 	case MMSPX_CH: return launch_ch_prec<PREC, 0>(g, p, a, b, st, t, nsteps);
 	case MMSPX_CH_DW: return launch_ch_prec<PREC, 1>(g, p, a, b, st, t, nsteps);
@@ -1373,6 +1354,7 @@ int fused_steps_per_launch(int model, const TuneChoice& t)
 {
 	if ((model == MMSPX_AC || model == MMSPX_CH || model == MMSPX_CH_DW) && (t.opt == 13 || t.opt == 14))
 		return steps2d_max_steps(model, t.opt);
+	if ((model == MMSPX_AC || model == MMSPX_CH || model == MMSPX_CH_DW) && t.opt == 15) return march4_max_steps(model);
 	if (model == MMSPX_AC && t.tz == kTbCols) return std::max(1, std::min(t.chunk, kTbMaxSteps));
 	if ((model == MMSPX_CH || model == MMSPX_CH_DW) && (t.opt == 6 || t.opt == 7)) return 2;
 	if ((model == MMSPX_GG || model == MMSPX_ZENER) && t.opt >= 9 && t.opt <= 11) return 2;

@@ -1,0 +1,106 @@
+// kernels_march4.hip -- the 3-D four-level march (march4.hpp): its FP64 form,
+// dispatch and tile choice (tile body 15).
+#include <algorithm>
+
+#include "march4_launch.hpp"
+
+namespace mmspx {
+
+int launch_march4_f32(const Geom& g, const ModelParams& p, const void* a, void* b, hipStream_t st, const TuneChoice& t,
+                      int nsteps);
+
+bool march4_supported(const Geom& g, int prec, int model)
+{
+	if (g.dim != 3 || (prec != MMSPX_F64 && prec != MMSPX_F32)) return false;
+	if (model != MMSPX_AC && model != MMSPX_CH && model != MMSPX_CH_DW) return false;
+	// byte offsets inside a plane are 32 bits
+	if ((int64_t)g.n[1] * g.n[2] >= (int64_t)1 << 28) return false;
+	for (int k = 0; k < 3; k++)
+		if (g.b0[k] != MMSPX_PERIODIC || g.b1[k] != MMSPX_PERIODIC) return false;
+	return true;
+}
+
+int march4_max_steps(int model) { return model == MMSPX_AC ? 4 : 2; }
+
+static const int kTiles[2][5][2] = {{{26, 52}, {16, 64}, {32, 32}, {16, 32}, {16, 16}},
+                                    {{32, 64}, {26, 52}, {32, 32}, {16, 32}, {16, 16}}};
+
+bool march4_tile_known(int prec, int ty, int tz)
+{
+	for (auto& t : kTiles[prec == MMSPX_F64 ? 0 : 1])
+		if (t[0] == ty && t[1] == tz) return true;
+	return false;
+}
+
+// Tile and chunk by a cost model: a workgroup of a chunk of c planes takes
+// c + 6 iterations (the march starts three planes early and ends three late);
+// tau is the time of one iteration when 1, 2, .. workgroups share a CU
+// (microseconds, Cahn-Hilliard; the last entry is how many fit), a launch
+// takes full rounds of 256 CUs and one of what is left. Fitted to a sweep of
+// chunks of 3 to 64 planes on 14 grids from 32^3 to 256^3, odd ones among
+// them. Against the former defaults (us per step): Allen-Cahn FP64 64^3 4.4
+// -> 3.3, 150 x 203 x 97 17.4 -> 7.7, 256^3 31.6 -> 27.4; FP32 150 x 203 x 97
+// 12.2 -> 5.2, 256^3 19.0 -> 13.4; Cahn-Hilliard FP64 64^3 8.0 -> 5.8, 150 x
+// 203 x 97 19.3 -> 12.1, 256^3 46.4 -> 42.1; FP32 150 x 203 x 97 13.9 -> 9.9,
+// 256^3 29.1 -> 24.3. The two-step register queues on 32 x 32 tiles (body 7)
+// stay where they are faster: FP64 Cahn-Hilliard on grids that 32 x 32 tiles
+// and their chunks divide into one round (128^3 9.6 against 10.6).
+bool march4_choice(const Geom& g, int prec, int model, TuneChoice* out)
+{
+	if (!march4_supported(g, prec, model)) return false;
+	constexpr double kCUs = 256;
+	static const double tau[2][5][6] = {
+	    {{1.45}, {1.36}, {1.36}, {1.00, 1.51}, {0.92, 1.10, 1.30, 1.51}},
+	    {{1.31}, {1.08, 1.64}, {1.05, 1.41}, {0.79, 1.00, 1.26, 1.52}, {0.77, 0.86, 0.96, 1.06, 1.16, 1.26}}};
+	const int f = prec == MMSPX_F64 ? 0 : 1;
+	auto time = [&](int64_t tiles, int c, const double* ta) {
+		int cap = 0;
+		while (cap < 6 && ta[cap] > 0.0) cap++;
+		const int64_t wgs = tiles * ((g.n[0] + c - 1) / c), round = (int64_t)(kCUs * cap);
+		const int64_t rest = wgs % round;
+		return (c + 6) * ((double)(wgs / round) * ta[cap - 1] + (rest ? ta[(int)((rest + 255) / 256) - 1] : 0.0));
+	};
+	double best = 1e300;
+	for (int k = 0; k < 5; k++) {
+		const int ty = kTiles[f][k][0], tz = kTiles[f][k][1];
+		const int64_t tiles = (int64_t)((g.n[1] + ty - 1) / ty) * ((g.n[2] + tz - 1) / tz);
+		for (int c = 3; c <= 64; c++) {
+			const double t = time(tiles, c, tau[f][k]);
+			if (t < best) {
+				best = t;
+				*out = TuneChoice{2, ty, tz, c, 15};
+			}
+		}
+	}
+	if (f == 0 && model != MMSPX_AC) {
+		static const double queues[6] = {1.25};
+		const int64_t tiles = (int64_t)((g.n[1] + 31) / 32) * ((g.n[2] + 31) / 32);
+		for (int c : {6, 8, 12, 16, 24, 32, 48, 64})
+			if (time(tiles, c, queues) < best) return false;
+	}
+	return true;
+}
+
+int launch_march4(const Geom& g, int prec, const ModelParams& p, const void* a, void* b, hipStream_t st,
+                  const TuneChoice& t, int nsteps)
+{
+	if (!march4_supported(g, prec, p.model))
+		return fail(MMSPX_EUNSUPPORTED, "the four-level march takes periodic 3-D Allen-Cahn and Cahn-Hilliard grids in "
+		                                "the MMSPX_F64 and MMSPX_F32 forms");
+	if (t.chunk < 1 || nsteps < 1) return fail(MMSPX_EINVAL, "bad chunk or step count");
+	return prec == MMSPX_F64 ? launch_march4_prec<MMSPX_F64>(g, p, a, b, st, t, nsteps)
+	                         : launch_march4_f32(g, p, a, b, st, t, nsteps);
+}
+
+// The body mmspx_get_tile reports for a default the four-level march runs: the
+// pass it takes the place of (7 and 12 several steps per pass, 8 the plane
+// march, which Allen-Cahn reports where 64-node tile rows would pad the last
+// axis by more than an eighth).
+int march4_reported_body(const Geom& g, int model)
+{
+	if (model != MMSPX_AC) return 7;
+	const int pad = (g.n[2] + 63) / 64 * 64 - g.n[2];
+	return pad * 8 <= g.n[2] ? 12 : 8;
+}
+
+}  // namespace mmspx
