@@ -4,8 +4,12 @@
 // many small solves that way leaves an MI355X idle. Here every member's tiles
 // go into one device work list and one persistent launch per step walks it
 // (workgroups take items blockIdx.x, blockIdx.x + gridDim.x, ...), whatever the
-// members' extents. Multi-step runs are captured once into a hipGraph (one
-// graph per starting parity, since each launch's arguments name the source
+// members' extents. By default Allen-Cahn and Cahn-Hilliard members whose axes
+// are periodic on both sides or on neither run the multi-step kernels
+// (kernels_batch_steps.hip), one launch per several steps: 32 uneven
+// Allen-Cahn members in FP32 took 21 us per step on the one-step strips, the
+// former default, and take 5. Multi-step runs are captured into a hipGraph (one
+// graph per starting parities, since each launch's arguments name the source
 // buffer) and replayed. The tile bodies are those of the single-grid kernels
 // (tiles.hpp), so each member's bits equal a single-grid run's.
 //
@@ -173,11 +177,16 @@ void member_items(int m, const Geom& g, int model, const BatchTile& t, std::vect
 {
 	const int nx = g.n[0];
 	if ((model == MMSPX_CH || model == MMSPX_CH_DW) && g.dim == 3) {
-		const int chunk = t.chunk3;
+		const int chunk = t.chunk3, ty = t.y3 > 0 ? t.y3 : kCh3TY, tz = t.z3 > 0 ? t.z3 : kCh3TZ;
 		for (int xb = 0; xb < nx; xb += chunk)
-			for (int y0 = 0; y0 < g.n[1]; y0 += kCh3TY)
-				for (int z0 = 0; z0 < g.n[2]; z0 += kCh3TZ)
-					out3.push_back(BItem{m, y0, z0, xb, std::min(xb + chunk, nx)});
+			for (int y0 = 0; y0 < g.n[1]; y0 += ty)
+				for (int z0 = 0; z0 < g.n[2]; z0 += tz) out3.push_back(BItem{m, y0, z0, xb, std::min(xb + chunk, nx)});
+		return;
+	}
+	if (t.lv > 0) {  // multi-step wave strips
+		for (int xb = 0; xb < nx; xb += t.chunk)
+			for (int c0 = 0; c0 < g.n[1]; c0 += 64 - 2 * t.lv)
+				out2.push_back(BItem{m, 0, c0, xb, std::min(xb + t.chunk, nx)});
 		return;
 	}
 	// 2-D: strips of the contiguous axis (axis 1). The strip bodies take the
@@ -250,18 +259,18 @@ static void launch_ch3(bool dw, const BMember* mem, const BItem* items, int n, i
 }
 
 template <int PREC>
-static void launch_prec(int model, int fields, const BatchTile& t, const BMember* mem, const BItem* l2, int n2,
-                        const BItem* l3, int n3, int parity, int cus, hipStream_t st, int nsteps)
+static void launch_prec2(int model, int fields, const BatchTile& t, const BMember* mem, const BItem* l2, int n2,
+                         int parity, int cus, hipStream_t st, int nsteps)
 {
-	if (n2 > 0 && model == MMSPX_AC && t.tb > 0) {
+	if (model == MMSPX_AC && t.tb > 0) {
 		const int blocks = std::max(1, std::min(n2, cus * t.bpc));
 		hipLaunchKernelGGL((ac_batch_tb<PREC>), dim3(blocks), dim3(256), 0, st, mem, l2, n2, parity, nsteps);
-	} else if (n2 > 0 && model == MMSPX_AC && t.cells > 0) {
+	} else if (model == MMSPX_AC && t.cells > 0) {
 		hipLaunchKernelGGL((ac_batch_cells<PREC>), dim3(n2), dim3(256), 0, st, mem, l2, parity);
-	} else if (n2 > 0 && (model == MMSPX_CH || model == MMSPX_CH_DW) && t.tz == kChWaveOut) {
+	} else if ((model == MMSPX_CH || model == MMSPX_CH_DW) && t.tz == kChWaveOut) {
 		const int blocks = std::max(1, std::min((n2 + 3) / 4, cus * t.bpc));
 		launch_ch2_waves<PREC>(model, mem, l2, n2, parity, blocks, st);
-	} else if (n2 > 0) {
+	} else {
 		const int blocks = std::max(1, std::min(n2, cus * t.bpc));
 		if (t.tz == 64)
 			launch_strips<PREC, 64>(model, fields, mem, l2, n2, parity, blocks, st);
@@ -270,25 +279,75 @@ static void launch_prec(int model, int fields, const BatchTile& t, const BMember
 		else
 			launch_strips<PREC, 256>(model, fields, mem, l2, n2, parity, blocks, st);
 	}
-	if (n3 > 0) {
-		const int blocks = std::max(1, std::min(n3, cus * t.bpc));
-		launch_ch3<PREC>(model == MMSPX_CH_DW, mem, l3, n3, parity, blocks, st);
+}
+
+template <int PREC>
+static void launch_prec(int model, int fields, const BatchTile& t, const BMember* mem, const BItem* items, int n, int dim,
+                        int parity, int cus, hipStream_t st, int nsteps)
+{
+	if (dim == 3)
+		launch_ch3<PREC>(model == MMSPX_CH_DW, mem, items, n, parity, std::max(1, std::min(n, cus * t.bpc)), st);
+	else
+		launch_prec2<PREC>(model, fields, t, mem, items, n, parity, cus, st, nsteps);
+}
+
+int batch_steps_per_pass(int model, const BatchTile& t, int dim)
+{
+	if (dim == 3) return t.y3 > 0 ? march4_max_steps(model) : 1;
+	if (t.lv > 0) return steps2d_max_steps(model, t.lv == 8 ? 13 : 14);
+	return t.tb > 0 ? std::min(t.tb, kTbMaxSteps) : 1;
+}
+
+void batch_multi_step_choice(int model, int prec, const Geom* const* g, int count, BatchTile* t)
+{
+	std::vector<const Geom*> g2, g3;
+	bool edges = false;
+	for (int m = 0; m < count; m++) {
+		if (g[m]->dim == 3) {
+			if (!march4_supported(*g[m], prec, model)) return;
+			g3.push_back(g[m]);
+		} else {
+			if (!steps2d_supported(*g[m], prec, model)) return;
+			for (int k = 0; k < 2; k++) edges |= g[m]->b0[k] != MMSPX_PERIODIC;
+			g2.push_back(g[m]);
+		}
+	}
+	if (!g2.empty()) {
+		const TuneChoice c = steps2d_choice_many(g2.data(), (int)g2.size(), prec, model);
+		t->lv = c.opt == 13 ? 8 : 4;
+		t->chunk = c.chunk;
+		t->edges = edges;
+	}
+	if (!g3.empty()) {
+		const TuneChoice c = march4_choice_many(g3.data(), (int)g3.size(), prec);
+		t->y3 = c.ty;
+		t->z3 = c.tz;
+		t->chunk3 = c.chunk;
 	}
 }
 
-int launch_batch_step(int model, int prec, int fields, const BatchTile& t, const BMember* mem, const BItem* l2, int n2,
-                      const BItem* l3, int n3, int parity, int cus, hipStream_t st, int64_t* launches, int nsteps)
+int launch_batch_pass(int model, int prec, int fields, const BatchTile& t, const BMember* mem, const BItem* items, int n,
+                      int dim, int parity, int cus, hipStream_t st, int64_t* launches, int nsteps)
 {
-	if (nsteps < 1 || nsteps > std::max(1, std::min(t.tb, kTbMaxSteps)))
+	if (n <= 0) return 0;
+	if (nsteps < 1 || nsteps > batch_steps_per_pass(model, t, dim))
 		return fail(MMSPX_EINVAL, "steps per pass exceed what the batch tile takes");
-	switch (prec) {
-	case MMSPX_F64: launch_prec<MMSPX_F64>(model, fields, t, mem, l2, n2, l3, n3, parity, cus, st, nsteps); break;
-	case MMSPX_F32: launch_prec<MMSPX_F32>(model, fields, t, mem, l2, n2, l3, n3, parity, cus, st, nsteps); break;
-	case MMSPX_F32REF: launch_prec<MMSPX_F32REF>(model, fields, t, mem, l2, n2, l3, n3, parity, cus, st, nsteps); break;
-	default: return fail(MMSPX_EINVAL, "unknown precision");
+	int rc = 0;
+	if (dim == 3 && t.y3 > 0) {
+		rc = launch_batch_march4(model, prec, t, mem, items, n, parity, st, nsteps);
+	} else if (dim == 2 && t.lv > 0) {
+		rc = launch_batch_steps2d(model, prec, t, mem, items, n, parity, st, nsteps);
+	} else {
+		switch (prec) {
+		case MMSPX_F64: launch_prec<MMSPX_F64>(model, fields, t, mem, items, n, dim, parity, cus, st, nsteps); break;
+		case MMSPX_F32: launch_prec<MMSPX_F32>(model, fields, t, mem, items, n, dim, parity, cus, st, nsteps); break;
+		case MMSPX_F32REF: launch_prec<MMSPX_F32REF>(model, fields, t, mem, items, n, dim, parity, cus, st, nsteps); break;
+		default: return fail(MMSPX_EINVAL, "unknown precision");
+		}
 	}
+	if (rc) return rc;
 	MMSPX_HIP(hipGetLastError());
-	*launches += (n2 > 0) + (n3 > 0);
+	*launches += 1;
 	return 0;
 }
 
@@ -335,10 +394,10 @@ struct mmspx_batch {
 	bool tuned = false;
 	int cus = 256;
 	int64_t steps_done = 0, launches = 0;
-	int64_t passes_done = 0;  // launches per item list so far: the buffer parity
+	int64_t passes2 = 0, passes3 = 0;  // passes over the 2-D and 3-D items so far: the buffer parities
 	hipStream_t st = nullptr;
 	hipEvent_t e0 = nullptr, e1 = nullptr;
-	hipGraphExec_t graph[2] = {nullptr, nullptr};
+	hipGraphExec_t graph[4] = {};  // by the buffer parities they start from, built when first needed
 	int graph_steps = 0;
 	double* part = nullptr;
 	double* part_host = nullptr;
@@ -377,8 +436,8 @@ static int upload_plan(mmspx_batch* b)
 			return fail(MMSPX_ENOMEM, "device allocation failed (work list)");
 		b->items_cap = need;
 	}
-	std::vector<BItem> all = xcd_order(l2);
-	const std::vector<BItem> o3 = xcd_order(l3);
+	std::vector<BItem> all = b->tile.lv > 0 ? l2 : xcd_order(l2);
+	const std::vector<BItem> o3 = b->tile.y3 > 0 ? l3 : xcd_order(l3);
 	all.insert(all.end(), o3.begin(), o3.end());
 	MMSPX_HIP(hipMemcpyAsync(b->d_items, all.data(), sizeof(BItem) * all.size(), hipMemcpyHostToDevice, b->st));
 	MMSPX_HIP(hipMemcpyAsync(b->d_mem, mem.data(), sizeof(BMember) * mem.size(), hipMemcpyHostToDevice, b->st));
@@ -389,53 +448,48 @@ static int upload_plan(mmspx_batch* b)
 	return 0;
 }
 
-static int steps_per_pass(const mmspx_batch* b) { return b->tile.tb > 0 ? std::min(b->tile.tb, kTbMaxSteps) : 1; }
-
-static int enqueue_steps(mmspx_batch* b, int steps)
+// Queues `steps` steps of every member: passes over the 2-D items, then over
+// the 3-D ones; p2 and p3 count the passes (the buffer parities).
+static int enqueue_passes(mmspx_batch* b, int steps, int64_t& p2, int64_t& p3, int64_t* launches)
 {
-	const int spp = steps_per_pass(b);
-	for (int left = steps; left > 0;) {
-		const int n = std::min(left, spp);
-		const int parity = (int)(b->passes_done & 1);
-		int rc = launch_batch_step(b->model, b->prec, b->fields, b->tile, b->d_mem, b->d_items, b->n2,
-		                           b->d_items + b->n2, b->n3, parity, b->cus, b->st, &b->launches, n);
-		if (rc) return rc;
-		b->passes_done += 1;
-		b->steps_done += n;
-		left -= n;
+	for (int dim = 2; dim <= 3; dim++) {
+		const int n = dim == 2 ? b->n2 : b->n3, spp = batch_steps_per_pass(b->model, b->tile, dim);
+		const BItem* items = b->d_items + (dim == 2 ? 0 : b->n2);
+		int64_t& p = dim == 2 ? p2 : p3;
+		for (int left = steps; n > 0 && left > 0; p++) {
+			const int k = std::min(left, spp);
+			int rc = launch_batch_pass(b->model, b->prec, b->fields, b->tile, b->d_mem, items, n, dim, (int)(p & 1), b->cus,
+			                           b->st, launches, k);
+			if (rc) return rc;
+			left -= k;
+		}
 	}
 	return 0;
 }
 
-static int graph_passes(const mmspx_batch* b, int gsteps) { return (gsteps + steps_per_pass(b) - 1) / steps_per_pass(b); }
-
-static int build_graphs(mmspx_batch* b, int gsteps)
+static int enqueue_steps(mmspx_batch* b, int steps)
 {
-	drop_graphs(b);
-	const int spp = steps_per_pass(b);
-	for (int start = 0; start < 2; start++) {
-		hipGraph_t graph = nullptr;
-		MMSPX_HIP(hipStreamBeginCapture(b->st, hipStreamCaptureModeThreadLocal));
-		int64_t dummy = 0;
-		int rc = 0;
-		int k = 0;
-		for (int left = gsteps; left > 0 && rc == 0; k++) {
-			const int n = std::min(left, spp);
-			rc = launch_batch_step(b->model, b->prec, b->fields, b->tile, b->d_mem, b->d_items, b->n2, b->d_items + b->n2,
-			                       b->n3, (start + k) & 1, b->cus, b->st, &dummy, n);
-			left -= n;
-		}
-		hipError_t e = hipStreamEndCapture(b->st, &graph);
-		if (rc) {
-			if (graph) (void)hipGraphDestroy(graph);
-			return rc;
-		}
-		if (e != hipSuccess) return fail(MMSPX_EDEVICE, std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
-		e = hipGraphInstantiate(&b->graph[start], graph, nullptr, nullptr, 0);
-		(void)hipGraphDestroy(graph);
-		if (e != hipSuccess) return fail(MMSPX_EDEVICE, std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
+	int rc = enqueue_passes(b, steps, b->passes2, b->passes3, &b->launches);
+	if (rc == 0) b->steps_done += steps;
+	return rc;
+}
+
+// The graph of gsteps steps that starts from the current buffer parities.
+static int build_graph(mmspx_batch* b, int gsteps, hipGraphExec_t* out)
+{
+	hipGraph_t graph = nullptr;
+	MMSPX_HIP(hipStreamBeginCapture(b->st, hipStreamCaptureModeThreadLocal));
+	int64_t dummy = 0, p2 = b->passes2, p3 = b->passes3;
+	int rc = enqueue_passes(b, gsteps, p2, p3, &dummy);
+	hipError_t e = hipStreamEndCapture(b->st, &graph);
+	if (rc) {
+		if (graph) (void)hipGraphDestroy(graph);
+		return rc;
 	}
-	b->graph_steps = gsteps;
+	if (e != hipSuccess) return fail(MMSPX_EDEVICE, std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
+	e = hipGraphInstantiate(out, graph, nullptr, nullptr, 0);
+	(void)hipGraphDestroy(graph);
+	if (e != hipSuccess) return fail(MMSPX_EDEVICE, std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
 	return 0;
 }
 
@@ -445,18 +499,26 @@ static int batch_step_impl(mmspx_batch* b, int steps, int gsteps)
 	if (!b->params_set) return fail(MMSPX_EINVAL, "mmspx_batch_set_params has not been called");
 	if (gsteps > 0 && steps >= gsteps) {
 		if (b->graph_steps != gsteps) {
-			int rc = build_graphs(b, gsteps);
-			if (rc) return rc;
+			drop_graphs(b);
+			b->graph_steps = gsteps;
 		}
-		const int reps = steps / gsteps;
-		const int gp = graph_passes(b, gsteps);
-		for (int r = 0; r < reps; r++) {
-			MMSPX_HIP(hipGraphLaunch(b->graph[b->passes_done & 1], b->st));
+		auto passes = [&](int dim) {
+			const int spp = batch_steps_per_pass(b->model, b->tile, dim);
+			return (dim == 2 ? b->n2 : b->n3) > 0 ? (gsteps + spp - 1) / spp : 0;
+		};
+		const int g2 = passes(2), g3 = passes(3);
+		for (; steps >= gsteps; steps -= gsteps) {
+			hipGraphExec_t& gx = b->graph[(b->passes2 & 1) * 2 + (b->passes3 & 1)];
+			if (!gx) {
+				int rc = build_graph(b, gsteps, &gx);
+				if (rc) return rc;
+			}
+			MMSPX_HIP(hipGraphLaunch(gx, b->st));
 			b->steps_done += gsteps;
-			b->passes_done += gp;
-			b->launches += (int64_t)gp * ((b->n2 > 0) + (b->n3 > 0));
+			b->passes2 += g2;
+			b->passes3 += g3;
+			b->launches += g2 + g3;
 		}
-		steps -= reps * gsteps;
 	}
 	return enqueue_steps(b, steps);
 }
@@ -522,6 +584,11 @@ int mmspx_batch_create(const mmspx_desc* descs, int count, int model, mmspx_batc
 	b->params.assign(count, ModelParams{});
 	// Cahn-Hilliard: 2-D members by wave strips (faster than the LDS row strips)
 	if (model == MMSPX_CH || model == MMSPX_CH_DW) b->tile = BatchTile{kChWaveOut, 8, 16, 8, 0};
+	{
+		std::vector<const Geom*> gs;
+		for (const Geom& g : b->geom) gs.push_back(&g);
+		batch_multi_step_choice(model, b->prec, gs.data(), count, &b->tile);
+	}
 	b->cus = device_cus();
 	b->arena_bytes = total;
 	const size_t red = (size_t)b->fields * 2 * kRedBlocks * sizeof(double);
@@ -543,7 +610,8 @@ int mmspx_batch_create(const mmspx_desc* descs, int count, int model, mmspx_batc
 	return 0;
 }
 
-static void* cur_buf(mmspx_batch* b, int m) { return b->arena + b->off[m] + ((b->passes_done & 1) ? b->bytes[m] : 0); }
+static bool odd_passes(const mmspx_batch* b, int m) { return ((b->geom[m].dim == 3 ? b->passes3 : b->passes2) & 1) != 0; }
+static void* cur_buf(mmspx_batch* b, int m) { return b->arena + b->off[m] + (odd_passes(b, m) ? b->bytes[m] : 0); }
 
 int mmspx_batch_upload(mmspx_batch* b, int m, const void* host, int layout)
 {
@@ -554,7 +622,7 @@ int mmspx_batch_upload(mmspx_batch* b, int m, const void* host, int layout)
 	if (g.fields == 1 || layout == MMSPX_FIELD_MAJOR) {
 		MMSPX_HIP(hipMemcpyAsync(dst, host, n, hipMemcpyHostToDevice, b->st));
 	} else {
-		void* spare = b->arena + b->off[m] + ((b->passes_done & 1) ? 0 : b->bytes[m]);
+		void* spare = b->arena + b->off[m] + (odd_passes(b, m) ? 0 : b->bytes[m]);
 		MMSPX_HIP(hipMemcpyAsync(spare, host, n, hipMemcpyHostToDevice, b->st));
 		int rc = launch_transpose(spare, dst, g.nodes, g.fields, b->prec == MMSPX_F64 ? 8 : 4, true, b->st);
 		if (rc) return rc;
@@ -572,7 +640,7 @@ int mmspx_batch_download(mmspx_batch* b, int m, void* host, int layout)
 	if (g.fields == 1 || layout == MMSPX_FIELD_MAJOR) {
 		MMSPX_HIP(hipMemcpyAsync(host, src, n, hipMemcpyDeviceToHost, b->st));
 	} else {
-		void* spare = b->arena + b->off[m] + ((b->passes_done & 1) ? 0 : b->bytes[m]);
+		void* spare = b->arena + b->off[m] + (odd_passes(b, m) ? 0 : b->bytes[m]);
 		int rc = launch_transpose(src, spare, g.nodes, g.fields, b->prec == MMSPX_F64 ? 8 : 4, false, b->st);
 		if (rc) return rc;
 		MMSPX_HIP(hipMemcpyAsync(host, spare, n, hipMemcpyDeviceToHost, b->st));
@@ -640,7 +708,7 @@ int mmspx_batch_set_tile(mmspx_batch* b, int tz, int chunk, int blocks_per_cu, i
 	if (tz == kTbCols) {  // temporal blocks: chunk = steps per pass
 		if (b->model != MMSPX_AC || !all_members_periodic(b) || chunk < 1 || chunk > kTbMaxSteps || blocks_per_cu < 1)
 			return fail(MMSPX_EINVAL, "temporal blocks: periodic Allen-Cahn members, 1..8 steps per pass");
-		BatchTile t{tz, 32, b->tile.chunk3, blocks_per_cu, 0};
+		BatchTile t{tz, 32, b->tile.y3 > 0 ? 16 : b->tile.chunk3, blocks_per_cu, 0};
 		t.tb = chunk;
 		b->tile = t;
 		return upload_plan(b);
@@ -650,7 +718,7 @@ int mmspx_batch_set_tile(mmspx_batch* b, int tz, int chunk, int blocks_per_cu, i
 	    cells < 0 || (cells > 0 && b->model != MMSPX_AC))
 		return fail(MMSPX_EINVAL, "strip width 64/128/256 (60: Cahn-Hilliard wave strips), positive rows and "
 		                          "workgroups; cell runs for Allen-Cahn only");
-	b->tile = BatchTile{tz, chunk, b->tile.chunk3, blocks_per_cu, cells};
+	b->tile = BatchTile{tz, chunk, b->tile.y3 > 0 ? 16 : b->tile.chunk3, blocks_per_cu, cells};
 	return upload_plan(b);
 }
 
@@ -658,9 +726,9 @@ int mmspx_batch_get_tile(const mmspx_batch* b, int* tz, int* chunk, int* blocks_
 {
 	if (!b) return fail(MMSPX_EINVAL, "null batch");
 	const BatchTile& t = b->tile;
-	if (tz) *tz = t.tb > 0 ? kTbCols : t.cells > 0 ? 0 : t.tz;
+	if (tz) *tz = t.lv > 0 ? 64 - 2 * t.lv : t.tb > 0 ? kTbCols : t.cells > 0 ? 0 : t.tz;
 	if (chunk) *chunk = t.tb > 0 ? t.tb : t.cells > 0 ? t.cells : t.chunk;
-	if (blocks_per_cu) *blocks_per_cu = t.cells > 0 ? 0 : t.bpc;
+	if (blocks_per_cu) *blocks_per_cu = t.cells > 0 || t.lv > 0 ? 0 : t.bpc;
 	return b->tuned ? 1 : 0;
 }
 
@@ -676,9 +744,10 @@ int mmspx_batch_autotune(mmspx_batch* b, int trial_steps, char* report, size_t r
 		b->staging_bytes = b->arena_bytes;
 	}
 	MMSPX_HIP(hipMemcpyAsync(b->staging, b->arena, b->arena_bytes, hipMemcpyDeviceToDevice, b->st));
-	const int64_t steps0 = b->steps_done, passes0 = b->passes_done;
+	const int64_t steps0 = b->steps_done, p2 = b->passes2, p3 = b->passes3;
 	const BatchTile keep = b->tile;
 	std::vector<BatchTile> cand;
+	if (b->tile.lv > 0 || b->tile.y3 > 0) cand.push_back(b->tile);  // the multi-step kernels as chosen
 	for (int tz : {64, 128, 256})
 		for (int chunk : {16, 32, 64, 128})
 			for (int bpc : {4, 8, 16}) cand.push_back(BatchTile{tz, chunk, 16, bpc, 0});
@@ -701,8 +770,9 @@ int mmspx_batch_autotune(mmspx_batch* b, int trial_steps, char* report, size_t r
 	for (const BatchTile& t : cand) {
 		b->tile = t;
 		rc = upload_plan(b);
-		// temporal blocks are timed over whole passes
-		const int steps = t.tb > 0 ? std::max(trial_steps, 2 * t.tb) / t.tb * t.tb : trial_steps;
+		// multi-step passes are timed over whole passes
+		const int spp = std::max(batch_steps_per_pass(b->model, t, 2), batch_steps_per_pass(b->model, t, 3));
+		const int steps = spp > 1 ? std::max(trial_steps, 2 * spp) / spp * spp : trial_steps;
 		if (rc == 0) rc = enqueue_steps(b, 2);
 		double sec = 0.0;
 		if (rc == 0) rc = mmspx_batch_step_timed(b, steps, 0, &sec);
@@ -710,7 +780,7 @@ int mmspx_batch_autotune(mmspx_batch* b, int trial_steps, char* report, size_t r
 		sec = sec / steps * trial_steps;
 		char line[160];
 		std::snprintf(line, sizeof line, "tz=%d chunk=%d blocks_per_cu=%d cells=%d steps_per_pass=%d us_per_step=%.2f\n",
-		              t.tz, t.chunk, t.bpc, t.cells, t.tb, sec / trial_steps * 1e6);
+		              t.lv > 0 ? 64 - 2 * t.lv : t.tz, t.chunk, t.bpc, t.cells, spp > 1 ? spp : 0, sec / trial_steps * 1e6);
 		rep += line;
 		if (sec < best) {
 			best = sec;
@@ -719,7 +789,8 @@ int mmspx_batch_autotune(mmspx_batch* b, int trial_steps, char* report, size_t r
 	}
 	b->tile = rc ? keep : best_t;
 	b->steps_done = steps0;
-	b->passes_done = passes0;
+	b->passes2 = p2;
+	b->passes3 = p3;
 	int rc2 = upload_plan(b);
 	if (hipMemcpyAsync(b->arena, b->staging, b->arena_bytes, hipMemcpyDeviceToDevice, b->st) != hipSuccess ||
 	    hipStreamSynchronize(b->st) != hipSuccess)

@@ -166,6 +166,7 @@ bool march4_supported(const Geom& g, int prec, int model);
 int march4_max_steps(int model);
 bool march4_tile_known(int prec, int ty, int tz);
 bool march4_choice(const Geom& g, int prec, int model, TuneChoice* out);
+TuneChoice march4_choice_many(const Geom* const* g, int count, int prec);  // one launch over all of them
 int march4_reported_body(const Geom& g, int model);
 int launch_march4(const Geom& g, int prec, const ModelParams& p, const void* a, void* b, hipStream_t st,
                   const TuneChoice& t, int nsteps);
@@ -175,6 +176,7 @@ int launch_march4(const Geom& g, int prec, const ModelParams& p, const void* a, 
 bool steps2d_supported(const Geom& g, int prec, int model);
 int steps2d_max_steps(int model, int body);
 bool steps2d_choice(const Geom& g, int prec, int model, TuneChoice* out);
+TuneChoice steps2d_choice_many(const Geom* const* g, int count, int prec, int model);  // one launch over all of them
 int launch_steps2d(const Geom& g, int prec, const ModelParams& p, const void* a, void* b, hipStream_t st, int body,
                    int chunk, int nsteps);
 int tile_candidates(const Geom& g, int prec, int model, TuneChoice* out, int max);

@@ -45,38 +45,59 @@ bool march4_tile_known(int prec, int ty, int tz)
 // 256^3 29.1 -> 24.3. The two-step register queues on 32 x 32 tiles (body 7)
 // stay where they are faster: FP64 Cahn-Hilliard on grids that 32 x 32 tiles
 // and their chunks divide into one round (128^3 9.6 against 10.6).
-bool march4_choice(const Geom& g, int prec, int model, TuneChoice* out)
+// us of one launch: `wgs` workgroups of c + 6 iterations, ta[n-1] us each with n to a CU
+static double march_time(int64_t wgs, int c, const double (&ta)[6])
 {
-	if (!march4_supported(g, prec, model)) return false;
-	constexpr double kCUs = 256;
+	int cap = 0;
+	while (cap < 6 && ta[cap] > 0.0) cap++;
+	const int64_t round = 256 * cap, rest = wgs % round;
+	return (c + 6) * ((double)(wgs / round) * ta[cap - 1] + (rest ? ta[(int)((rest + 255) / 256) - 1] : 0.0));
+}
+
+static int64_t march_wgs(const Geom& g, int ty, int tz, int c)
+{
+	return (int64_t)((g.n[1] + ty - 1) / ty) * ((g.n[2] + tz - 1) / tz) * ((g.n[0] + c - 1) / c);
+}
+
+static TuneChoice march_best(const Geom* const* g, int count, int prec, double* us)
+{
 	static const double tau[2][5][6] = {
 	    {{1.45}, {1.36}, {1.36}, {1.00, 1.51}, {0.92, 1.10, 1.30, 1.51}},
 	    {{1.31}, {1.08, 1.64}, {1.05, 1.41}, {0.79, 1.00, 1.26, 1.52}, {0.77, 0.86, 0.96, 1.06, 1.16, 1.26}}};
 	const int f = prec == MMSPX_F64 ? 0 : 1;
-	auto time = [&](int64_t tiles, int c, const double* ta) {
-		int cap = 0;
-		while (cap < 6 && ta[cap] > 0.0) cap++;
-		const int64_t wgs = tiles * ((g.n[0] + c - 1) / c), round = (int64_t)(kCUs * cap);
-		const int64_t rest = wgs % round;
-		return (c + 6) * ((double)(wgs / round) * ta[cap - 1] + (rest ? ta[(int)((rest + 255) / 256) - 1] : 0.0));
-	};
-	double best = 1e300;
+	TuneChoice out{2, 16, 32, 8, 15};
+	*us = 1e300;
 	for (int k = 0; k < 5; k++) {
 		const int ty = kTiles[f][k][0], tz = kTiles[f][k][1];
-		const int64_t tiles = (int64_t)((g.n[1] + ty - 1) / ty) * ((g.n[2] + tz - 1) / tz);
-		for (int c = 3; c <= 64; c++) {
-			const double t = time(tiles, c, tau[f][k]);
-			if (t < best) {
-				best = t;
-				*out = TuneChoice{2, ty, tz, c, 15};
+		for (int c = 3; c <= 64; c += count > 1 && c >= 8 ? 4 : 1) {
+			int64_t wgs = 0;
+			for (int m = 0; m < count; m++) wgs += march_wgs(*g[m], ty, tz, c);
+			const double t = march_time(wgs, c, tau[f][k]);
+			if (t < *us) {
+				*us = t;
+				out = TuneChoice{2, ty, tz, c, 15};
 			}
 		}
 	}
-	if (f == 0 && model != MMSPX_AC) {
+	return out;
+}
+
+TuneChoice march4_choice_many(const Geom* const* g, int count, int prec)
+{
+	double us;
+	return march_best(g, count, prec, &us);
+}
+
+bool march4_choice(const Geom& g, int prec, int model, TuneChoice* out)
+{
+	if (!march4_supported(g, prec, model)) return false;
+	const Geom* one = &g;
+	double us;
+	*out = march_best(&one, 1, prec, &us);
+	if (prec == MMSPX_F64 && model != MMSPX_AC) {
 		static const double queues[6] = {1.25};
-		const int64_t tiles = (int64_t)((g.n[1] + 31) / 32) * ((g.n[2] + 31) / 32);
 		for (int c : {6, 8, 12, 16, 24, 32, 48, 64})
-			if (time(tiles, c, queues) < best) return false;
+			if (march_time(march_wgs(g, 32, 32, c), c, queues) < us) return false;
 	}
 	return true;
 }

@@ -107,9 +107,8 @@ int steps2d_max_steps(int model, int body) { return (body == 13 ? 8 : 4) / (mode
 // 1024^2 6.00 -> 2.83, 4096^2 43.5 -> 21.4; FP32 1024^2 2.18 -> 1.36 and 4.69
 // -> 2.19; walls, FP64 407 x 756: Allen-Cahn 3.66 -> 1.69, Cahn-Hilliard
 // 4.17 -> 2.83. It was faster at every size tried, 17 x 49 to 4096^2.
-bool steps2d_choice(const Geom& g, int prec, int model, TuneChoice* out)
+TuneChoice steps2d_choice_many(const Geom* const* g, int count, int prec, int model)
 {
-	if (!steps2d_supported(g, prec, model)) return false;
 	constexpr double kT0 = 2.5, kSimds = 1024, kBytesPerUs = 5e6;
 	const bool f64 = prec == MMSPX_F64;
 	const double level = model == MMSPX_AC ? (f64 ? 0.054 : 0.040) : model == MMSPX_CH_DW ? (f64 ? 0.0375 : 0.033)
@@ -117,23 +116,38 @@ bool steps2d_choice(const Geom& g, int prec, int model, TuneChoice* out)
 	const double share = model == MMSPX_AC ? (f64 ? 0.72 : 0.56) : model == MMSPX_CH_DW ? (f64 ? 0.64 : 0.47)
 	                                                                                    : (f64 ? 0.68 : 0.50);
 	bool edges = false;
-	for (int k = 0; k < 2; k++) edges |= g.b0[k] != MMSPX_PERIODIC;
-	const double move = 2.0 * g.nodes * (f64 ? 8 : 4) / kBytesPerUs;
+	double nodes = 0.0;
+	for (int m = 0; m < count; m++) {
+		for (int k = 0; k < 2; k++) edges |= g[m]->b0[k] != MMSPX_PERIODIC;
+		nodes += g[m]->nodes;
+	}
+	const double move = 2.0 * nodes * (f64 ? 8 : 4) / kBytesPerUs;
+	TuneChoice out{2, 1, kSteps8Cols, 8, 13};
 	double best = 1e300;
 	for (int body = 13; body <= 14; body++) {
 		const int L = body == 13 ? 8 : 4, cols = 64 - 2 * L;
-		const double strips = (g.n[1] + cols - 1) / cols;
-		for (int c = 2; c <= 64; c++) {
-			double n = strips * ((g.n[0] + c - 1) / c) / kSimds;
+		for (int c = 2; c <= 64; c += count > 1 && c >= 8 ? 4 : 1) {
+			double waves = 0.0;
+			for (int m = 0; m < count; m++)
+				waves += (double)((g[m]->n[1] + cols - 1) / cols) * ((g[m]->n[0] + c - 1) / c);
+			double n = waves / kSimds;
 			n = n <= 4.0 ? std::ceil(n) : n + 0.5;
 			const double wave = level * (edges ? 1.0 + 0.045 * L : 1.0) * L * (c + L - 1) * std::max(1.0, 0.28 + share * n);
 			const double cost = (kT0 + std::max(wave, move) + 0.25 * std::min(wave, move)) / L;
 			if (cost < best) {
 				best = cost;
-				*out = TuneChoice{2, 1, cols, c, body};
+				out = TuneChoice{2, 1, cols, c, body};
 			}
 		}
 	}
+	return out;
+}
+
+bool steps2d_choice(const Geom& g, int prec, int model, TuneChoice* out)
+{
+	if (!steps2d_supported(g, prec, model)) return false;
+	const Geom* one = &g;
+	*out = steps2d_choice_many(&one, 1, prec, model);
 	return true;
 }
 

@@ -18,9 +18,9 @@
 //   * the worker advances resident requests in rounds. Each round takes the
 //     requests with the least remaining work until it holds enough nodes per
 //     step to fill the GPU (plus any request left out for too long); it lasts
-//     until one of them finishes or `chunk_steps` steps, and is one
-//     persistent launch per step over every member's tiles (2-D and 3-D
-//     members in two launches). 3-D members of 2^21 nodes or more fill the
+//     until one of them finishes or `chunk_steps` steps, in passes of several
+//     steps over every member's items (2-D and 3-D members, FP32 and FP64 ones
+//     in launches of their own). 3-D members of 2^21 nodes or more fill the
 //     GPU on their own: they run the single-grid kernels instead (for
 //     periodic Cahn-Hilliard two steps per pass), one launch per member and
 //     pass, on a second compute stream, so they overlap the batch launches
@@ -32,12 +32,10 @@
 //     round, takes the FP64 mass of the final state, copies it out and frees
 //     its buffers; only then is its memory counted free for admission.
 // Uploads and downloads therefore overlap the compute of the other requests.
-// A batched member's state after s steps sits in buf[s & 1], so joining
-// mid-stream or sitting out rounds needs no copy; a member on the single-grid
-// kernels keeps the index of the buffer holding its state (a two-step pass
-// swaps the buffers once). The tile bodies are the
-// single-grid kernels' (tiles.hpp): a request's result does not depend on what
-// else was resident.
+// A request keeps the index of the buffer holding its state (a pass swaps the
+// buffers once, whatever its steps), so joining mid-stream or sitting out
+// rounds needs no copy. The tile bodies are the single-grid kernels': a
+// request's result does not depend on what else was resident.
 #include <algorithm>
 #include <chrono>
 #include <condition_variable>
@@ -77,7 +75,7 @@ struct Request {
 	int idle_rounds = 0;             // rounds planned since it last advanced
 	bool solo = false;               // runs the single-grid kernels with `tile`
 	TuneChoice tile{};
-	int cur = 0;                     // solo: the buffer holding the state after `planned` steps
+	int cur = 0;                     // the buffer holding the state after `planned` steps
 	int in_rounds = 0;               // queued rounds that list it (under the server's mutex)
 	bool fetched = false;            // fetched while rounds still listed it: the worker deletes it
 	hipEvent_t ev_last = nullptr;    // recorded after its last round (or when dropped)
@@ -147,7 +145,6 @@ struct mmspx_server {
 	// worker-only state
 	std::vector<Request*> resident;
 	std::deque<Round> rounds;
-	int64_t gstep = 0;  // global steps queued so far
 	Slot slot[kSlots];
 	int next_slot = 0;
 
@@ -224,8 +221,7 @@ static void uploader_main(mmspx_server* sv)
 static int download_one(mmspx_server* sv, Request* r, std::vector<double>& part_host)
 {
 	MMSPX_HIP(hipStreamWaitEvent(sv->dst, r->ev_last, 0));
-	const int last = r->solo ? r->cur : (r->steps & 1);
-	const void* s = r->dev + (last ? r->bytes : 0);
+	const void* s = r->dev + (r->cur ? r->bytes : 0);
 	int rc = launch_reduce(r->g, r->prec, MMSPX_MASS, r->p, s, sv->dpart, sv->dst);
 	if (rc) return rc;
 	MMSPX_HIP(hipMemcpyAsync(part_host.data(), sv->dpart, part_host.size() * sizeof(double), hipMemcpyDeviceToHost,
@@ -324,10 +320,8 @@ static std::vector<Request*> pick_round(mmspx_server* sv)
 }
 
 // Plans one round over the picked members and queues it on the compute stream;
-// members whose last step it holds are handed to the downloader. A member's
-// state after s steps sits in buf[s & 1] (buf[0] holds the uploaded state),
-// so members that sat out rounds need no copy: the phase sent with each
-// round maps the launch parity onto the member's own step count.
+// members whose last step it holds are handed to the downloader. The phase
+// sent with each round is the buffer the member's state sits in.
 static int enqueue_round(mmspx_server* sv)
 {
 	std::vector<Request*> act = pick_round(sv);
@@ -339,12 +333,21 @@ static int enqueue_round(mmspx_server* sv)
 	// the pinned mirrors are rewritten below: the copy that read them last must be done
 	if (sl.used) MMSPX_HIP(hipEventSynchronize(sl.done));
 	// work lists per form: group 0 the server's precision, group 1 the FP64
-	// requests of an FP32 server; each group is one launch per step and kind
+	// requests of an FP32 server; each group takes its passes, 2-D members then
+	// 3-D ones, on the multi-step kernels where they take its members
+	const int form[2] = {sv->cfg.precision, MMSPX_F64};
+	BatchTile tile[2] = {sv->tile, sv->tile};
 	std::vector<BItem> l2[2], l3[2];
+	for (int k = 0; k < 2; k++) {
+		std::vector<const Geom*> gs;
+		for (const Request* r : act)
+			if (!r->solo && (r->prec != sv->cfg.precision) == (k == 1)) gs.push_back(&r->g);
+		if (!gs.empty()) batch_multi_step_choice(sv->cfg.model, form[k], gs.data(), (int)gs.size(), &tile[k]);
+	}
 	for (size_t m = 0; m < act.size(); m++) {
 		if (act[m]->solo) continue;
 		const int grp = act[m]->prec != sv->cfg.precision;
-		member_items((int)m, act[m]->g, sv->cfg.model, sv->tile, l2[grp], l3[grp]);
+		member_items((int)m, act[m]->g, sv->cfg.model, tile[grp], l2[grp], l3[grp]);
 	}
 	int n2[2], n3[2], off[2], total = 0;
 	for (int k = 0; k < 2; k++) {
@@ -362,26 +365,32 @@ static int enqueue_round(mmspx_server* sv)
 		bm.buf[1] = r->dev + r->bytes;
 		bm.g = r->g;
 		bm.p = r->p;
-		bm.phase = (int)((r->planned - sv->gstep) & 1);
+		bm.phase = r->cur;
 	}
 	for (int k = 0; k < 2; k++) {
-		const std::vector<BItem> o2 = xcd_order(l2[k]), o3 = xcd_order(l3[k]);
+		const std::vector<BItem> o2 = tile[k].lv > 0 ? l2[k] : xcd_order(l2[k]);
+		const std::vector<BItem> o3 = tile[k].y3 > 0 ? l3[k] : xcd_order(l3[k]);
 		std::copy(o2.begin(), o2.end(), sl.h_items + off[k]);
 		std::copy(o3.begin(), o3.end(), sl.h_items + off[k] + n2[k]);
 	}
 	MMSPX_HIP(hipMemcpyAsync(sl.d_mem, sl.h_mem, sizeof(BMember) * act.size(), hipMemcpyHostToDevice, sv->st));
 	MMSPX_HIP(hipMemcpyAsync(sl.d_items, sl.h_items, sizeof(BItem) * (size_t)total, hipMemcpyHostToDevice, sv->st));
 	int64_t launches = 0;
-	const int form[2] = {sv->cfg.precision, MMSPX_F64};
-	for (int k = 0; k < steps; k++) {
-		for (int grp = 0; grp < 2; grp++) {
-			if (n2[grp] + n3[grp] == 0) continue;
-			const BItem* it = sl.d_items + off[grp];
-			rc = launch_batch_step(sv->cfg.model, form[grp], 1, sv->tile, sl.d_mem, it, n2[grp], it + n2[grp], n3[grp],
-			                       (int)((sv->gstep + k) & 1), sv->cus, sv->st, &launches);
-			if (rc) return rc;
+	int passes[2][2];  // by group and dimension
+	for (int grp = 0; grp < 2; grp++) {
+		for (int dim = 2; dim <= 3; dim++) {
+			const int n = dim == 2 ? n2[grp] : n3[grp], spp = batch_steps_per_pass(sv->cfg.model, tile[grp], dim);
+			const BItem* it = sl.d_items + off[grp] + (dim == 2 ? 0 : n2[grp]);
+			passes[grp][dim - 2] = (steps + spp - 1) / spp;
+			for (int k = 0; n > 0 && k * spp < steps; k++) {
+				rc = launch_batch_pass(sv->cfg.model, form[grp], 1, tile[grp], sl.d_mem, it, n, dim, k & 1, sv->cus, sv->st,
+				                       &launches, std::min(spp, steps - k * spp));
+				if (rc) return rc;
+			}
 		}
 	}
+	for (Request* r : act)
+		if (!r->solo) r->cur ^= passes[r->prec != sv->cfg.precision][r->g.dim == 3 ? 1 : 0] & 1;
 	// the large 3-D members: their own single-grid launches
 	for (Request* r : act) {
 		if (!r->solo) continue;
@@ -406,7 +415,6 @@ static int enqueue_round(mmspx_server* sv)
 	}
 	MMSPX_HIP(hipEventRecord(sl.done, sv->st));
 	sl.used = true;
-	sv->gstep += steps;
 	std::vector<Request*> keep;
 	std::vector<IoJob> fin;
 	for (Request* r : sv->resident) r->idle_rounds += 1;
