@@ -240,6 +240,7 @@ void mmspx_destroy(mmspx_state* s)
 	if (s->ev1) (void)hipEventDestroy(s->ev1);
 	if (s->stream) (void)hipStreamDestroy(s->stream);
 	delete s;
+	staging_release();
 }
 
 int mmspx_create(const mmspx_desc* d, mmspx_state** out)
@@ -250,6 +251,7 @@ int mmspx_create(const mmspx_desc* d, mmspx_state** out)
 	if (rc) return rc;
 	mmspx_state* s = new (std::nothrow) mmspx_state();
 	if (!s) return fail(MMSPX_ENOMEM, "host allocation failed");
+	staging_retain();
 	s->desc = *d;
 	s->geom = make_geom(*d);
 	s->elem = d->precision == MMSPX_F64 ? 8 : 4;
@@ -288,11 +290,12 @@ int mmspx_upload(mmspx_state* s, const void* host, int layout)
 	if (!s || !host) return fail(MMSPX_EINVAL, "null argument");
 	if (layout != MMSPX_NODE_MAJOR && layout != MMSPX_FIELD_MAJOR) return fail(MMSPX_EINVAL, "unknown layout");
 	if (s->geom.fields == 1 || layout == MMSPX_FIELD_MAJOR) {
-		MMSPX_HIP(hipMemcpyAsync(s->cur, host, s->bytes, hipMemcpyHostToDevice, s->stream));
+		return copy_to_device(s->cur, host, s->bytes, s->stream);
 	} else {
 		// stage node-major in the spare buffer, transpose into the state
-		MMSPX_HIP(hipMemcpyAsync(s->nxt, host, s->bytes, hipMemcpyHostToDevice, s->stream));
-		int rc = launch_transpose(s->nxt, s->cur, s->geom.nodes, s->geom.fields, s->elem, true, s->stream);
+		int rc = copy_to_device(s->nxt, host, s->bytes, s->stream);
+		if (rc) return rc;
+		rc = launch_transpose(s->nxt, s->cur, s->geom.nodes, s->geom.fields, s->elem, true, s->stream);
 		if (rc) return rc;
 	}
 	MMSPX_HIP(hipStreamSynchronize(s->stream));
@@ -304,14 +307,11 @@ int mmspx_download(mmspx_state* s, void* host, int layout)
 	if (!s || !host) return fail(MMSPX_EINVAL, "null argument");
 	if (layout != MMSPX_NODE_MAJOR && layout != MMSPX_FIELD_MAJOR) return fail(MMSPX_EINVAL, "unknown layout");
 	if (s->geom.fields == 1 || layout == MMSPX_FIELD_MAJOR) {
-		MMSPX_HIP(hipMemcpyAsync(host, s->cur, s->bytes, hipMemcpyDeviceToHost, s->stream));
-	} else {
-		int rc = launch_transpose(s->cur, s->nxt, s->geom.nodes, s->geom.fields, s->elem, false, s->stream);
-		if (rc) return rc;
-		MMSPX_HIP(hipMemcpyAsync(host, s->nxt, s->bytes, hipMemcpyDeviceToHost, s->stream));
+		return copy_to_host(host, s->cur, s->bytes, s->stream);
 	}
-	MMSPX_HIP(hipStreamSynchronize(s->stream));
-	return 0;
+	int rc = launch_transpose(s->cur, s->nxt, s->geom.nodes, s->geom.fields, s->elem, false, s->stream);
+	if (rc) return rc;
+	return copy_to_host(host, s->nxt, s->bytes, s->stream);
 }
 
 int mmspx_set_variant(mmspx_state* s, int variant)
@@ -733,11 +733,14 @@ int mmspx_reduce(mmspx_state* s, int what, int model, const double* params, int 
 	} else {
 		return fail(MMSPX_EINVAL, "unknown reduction");
 	}
-	int rc = launch_reduce(s->geom, s->desc.precision, what, p, s->cur, s->part, s->stream);
-	if (rc) return rc;
+	// few fields: the kernel writes its partials to pinned host memory itself
+	// (8 KiB a field; a copy of its own took 6 us more on a 128^2 grid)
 	const int sets = what == MMSPX_MASS ? s->geom.fields : 1;
+	const bool direct = sets <= 4;
+	int rc = launch_reduce(s->geom, s->desc.precision, what, p, s->cur, direct ? s->part_host : s->part, s->stream);
+	if (rc) return rc;
 	const size_t bytes = (size_t)sets * 2 * kRedBlocks * sizeof(double);
-	MMSPX_HIP(hipMemcpyAsync(s->part_host, s->part, bytes, hipMemcpyDeviceToHost, s->stream));
+	if (!direct) MMSPX_HIP(hipMemcpyAsync(s->part_host, s->part, bytes, hipMemcpyDeviceToHost, s->stream));
 	MMSPX_HIP(hipStreamSynchronize(s->stream));
 	for (int j = 0; j < sets; j++) out[j] = sum_partials(s->part_host + (size_t)j * 2 * kRedBlocks, kRedBlocks);
 	if (what == MMSPX_ENERGY) out[0] *= s->geom.vol;

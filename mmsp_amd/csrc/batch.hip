@@ -540,6 +540,7 @@ void mmspx_batch_destroy(mmspx_batch* b)
 	if (b->e1) (void)hipEventDestroy(b->e1);
 	if (b->st) (void)hipStreamDestroy(b->st);
 	delete b;
+	staging_release();
 }
 
 int mmspx_batch_create(const mmspx_desc* descs, int count, int model, mmspx_batch** out)
@@ -581,6 +582,7 @@ int mmspx_batch_create(const mmspx_desc* descs, int count, int model, mmspx_batc
 		b->bytes.push_back(bytes);
 		total += 2 * bytes;
 	}
+	staging_retain();
 	b->params.assign(count, ModelParams{});
 	// Cahn-Hilliard: 2-D members by wave strips (faster than the LDS row strips)
 	if (model == MMSPX_CH || model == MMSPX_CH_DW) b->tile = BatchTile{kChWaveOut, 8, 16, 8, 0};
@@ -620,11 +622,12 @@ int mmspx_batch_upload(mmspx_batch* b, int m, const void* host, int layout)
 	const size_t n = (size_t)g.nodes * g.fields * (b->prec == MMSPX_F64 ? 8 : 4);
 	void* dst = cur_buf(b, m);
 	if (g.fields == 1 || layout == MMSPX_FIELD_MAJOR) {
-		MMSPX_HIP(hipMemcpyAsync(dst, host, n, hipMemcpyHostToDevice, b->st));
+		return copy_to_device(dst, host, n, b->st);
 	} else {
 		void* spare = b->arena + b->off[m] + (odd_passes(b, m) ? 0 : b->bytes[m]);
-		MMSPX_HIP(hipMemcpyAsync(spare, host, n, hipMemcpyHostToDevice, b->st));
-		int rc = launch_transpose(spare, dst, g.nodes, g.fields, b->prec == MMSPX_F64 ? 8 : 4, true, b->st);
+		int rc = copy_to_device(spare, host, n, b->st);
+		if (rc) return rc;
+		rc = launch_transpose(spare, dst, g.nodes, g.fields, b->prec == MMSPX_F64 ? 8 : 4, true, b->st);
 		if (rc) return rc;
 	}
 	MMSPX_HIP(hipStreamSynchronize(b->st));
@@ -638,15 +641,12 @@ int mmspx_batch_download(mmspx_batch* b, int m, void* host, int layout)
 	const size_t n = (size_t)g.nodes * g.fields * (b->prec == MMSPX_F64 ? 8 : 4);
 	void* src = cur_buf(b, m);
 	if (g.fields == 1 || layout == MMSPX_FIELD_MAJOR) {
-		MMSPX_HIP(hipMemcpyAsync(host, src, n, hipMemcpyDeviceToHost, b->st));
-	} else {
-		void* spare = b->arena + b->off[m] + (odd_passes(b, m) ? 0 : b->bytes[m]);
-		int rc = launch_transpose(src, spare, g.nodes, g.fields, b->prec == MMSPX_F64 ? 8 : 4, false, b->st);
-		if (rc) return rc;
-		MMSPX_HIP(hipMemcpyAsync(host, spare, n, hipMemcpyDeviceToHost, b->st));
+		return copy_to_host(host, src, n, b->st);
 	}
-	MMSPX_HIP(hipStreamSynchronize(b->st));
-	return 0;
+	void* spare = b->arena + b->off[m] + (odd_passes(b, m) ? 0 : b->bytes[m]);
+	int rc = launch_transpose(src, spare, g.nodes, g.fields, b->prec == MMSPX_F64 ? 8 : 4, false, b->st);
+	if (rc) return rc;
+	return copy_to_host(host, spare, n, b->st);
 }
 
 int mmspx_batch_set_params(mmspx_batch* b, const double* params, int np)
@@ -683,11 +683,14 @@ int mmspx_batch_reduce(mmspx_batch* b, int m, int what, double* out, int nout)
 	if (what == MMSPX_MASS && nout < g.fields) return fail(MMSPX_EINVAL, "mass needs one output per field");
 	if (what == MMSPX_ENERGY && nout < 1) return fail(MMSPX_EINVAL, "energy needs one output");
 	if (what != MMSPX_MASS && what != MMSPX_ENERGY) return fail(MMSPX_EINVAL, "unknown reduction");
-	int rc = launch_reduce(g, b->prec, what, b->params[m], cur_buf(b, m), b->part, b->st);
-	if (rc) return rc;
+	// few fields: partials straight to pinned host memory, as for a single state
 	const int sets = what == MMSPX_MASS ? g.fields : 1;
-	MMSPX_HIP(hipMemcpyAsync(b->part_host, b->part, (size_t)sets * 2 * kRedBlocks * sizeof(double),
-	                         hipMemcpyDeviceToHost, b->st));
+	const bool direct = sets <= 4;
+	int rc = launch_reduce(g, b->prec, what, b->params[m], cur_buf(b, m), direct ? b->part_host : b->part, b->st);
+	if (rc) return rc;
+	if (!direct)
+		MMSPX_HIP(hipMemcpyAsync(b->part_host, b->part, (size_t)sets * 2 * kRedBlocks * sizeof(double),
+		                         hipMemcpyDeviceToHost, b->st));
 	MMSPX_HIP(hipStreamSynchronize(b->st));
 	for (int j = 0; j < sets; j++) out[j] = sum_partials(b->part_host + (size_t)j * 2 * kRedBlocks, kRedBlocks);
 	if (what == MMSPX_ENERGY) out[0] *= g.vol;

@@ -159,6 +159,13 @@ int launch_transpose(const void* src, void* dst, int nodes, int fields, size_t e
                      hipStream_t st);
 int launch_convert(const void* src, int src_f64, void* dst, int dst_f64, int64_t n, hipStream_t st);
 int launch_copy(const void* src, void* dst, size_t bytes, hipStream_t st);
+// copies between the caller's host memory and the device, done on return
+// (transfer.hip); the pinned memory they go through lives while a state or
+// batch holds it
+int copy_to_host(void* dst, const void* src, size_t bytes, hipStream_t st);
+int copy_to_device(void* dst, const void* src, size_t bytes, hipStream_t st);
+void staging_retain();
+void staging_release();
 bool tile_known(const Geom& g, const TuneChoice& t);
 // 3-D four-level march (kernels_march4.hip), tile body 15: two Cahn-Hilliard
 // or four Allen-Cahn steps per pass on periodic grids
