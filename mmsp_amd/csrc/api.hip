@@ -467,8 +467,10 @@ int mmspx_set_tile(mmspx_state* s, int ty, int tz, int chunk)
 	if (s->geom.dim == 2 && ty > 1 && tz == kTbCols) opt = 3;
 	else if (s->geom.dim == 2 && ty > 1) opt = 1;
 	else if (s->geom.dim == 2 && s->tuned && s->tile.ty > 1) opt = 0;
-	// 1 x 48 and 1 x 56 name the 2-D multi-step wave strips
-	if (s->geom.dim == 2 && ty == 1 && (tz == kSteps8Cols || tz == kSteps4Cols)) opt = tz == kSteps8Cols ? 13 : 14;
+	// 1 x 48 and 1 x 56 name the 2-D multi-step wave strips (1 x 56 also the
+	// four-step field strips, where their body was chosen)
+	if (s->geom.dim == 2 && ty == 1 && (tz == kSteps8Cols || tz == kSteps4Cols))
+		opt = tz == kSteps8Cols ? 13 : s->tuned && s->tile.opt == 16 ? 16 : 14;
 	// 3-D two-step bodies: 32 x 32 tiles run body 7 only; body 6 runs 32 x 64
 	if (s->geom.dim == 3 && ty == 32 && tz == 32) opt = 7;
 	else if (s->geom.dim == 3 && s->tuned && s->tile.opt == 6 && ty == 32 && tz == 64) opt = 6;
@@ -487,8 +489,8 @@ int mmspx_set_tile(mmspx_state* s, int ty, int tz, int chunk)
 int mmspx_set_tile_options(mmspx_state* s, int body)
 {
 	if (!s) return fail(MMSPX_EINVAL, "null state");
-	if (body < 0 || body > 15 || (body == 3 && s->geom.dim != 3) ||
-	    ((body == 4 || body == 5 || (body >= 9 && body <= 11) || body == 13 || body == 14) &&
+	if (body < 0 || body > 16 || (body == 3 && s->geom.dim != 3) ||
+	    ((body == 4 || body == 5 || (body >= 9 && body <= 11) || body == 13 || body == 14 || body == 16) &&
 	     s->geom.dim != 2) ||
 	    (((body >= 6 && body <= 8) || body == 12 || body == 15) && s->geom.dim != 3))
 		return fail(MMSPX_EINVAL, "unknown tile body");

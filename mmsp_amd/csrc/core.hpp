@@ -177,6 +177,13 @@ TuneChoice march4_choice_many(const Geom* const* g, int count, int prec);  // on
 int march4_reported_body(const Geom& g, int model);
 int launch_march4(const Geom& g, int prec, const ModelParams& p, const void* a, void* b, hipStream_t st,
                   const TuneChoice& t, int nsteps);
+// 2-D four-step field strips (kernels_fields2d.hip), tile body 16: grain growth
+// and Zener pinning, strips of kSteps4Cols columns, `chunk` rows per workgroup
+constexpr int kFieldsSteps = 4;
+bool fields2d_supported(const Geom& g, int prec, int model);
+bool fields2d_choice(const Geom& g, int prec, int model, TuneChoice* out);
+int launch_fields2d(const Geom& g, int prec, const ModelParams& p, const void* a, void* b, hipStream_t st, int chunk,
+                    int nsteps);
 // 2-D multi-step wave strips (kernels_steps2d.hip): tile bodies 13 (strips of
 // 48 columns) and 14 (56), `chunk` rows per wave; a pass takes up to
 // steps2d_max_steps steps
