@@ -283,7 +283,8 @@ int mmspx_set_tile(mmspx_state* s, int ty, int tz, int chunk);
  * registers (their default). 3-D periodic Allen-Cahn and Cahn-Hilliard
  * (deterministic chemical potentials) in the same forms: 15 is the four-level
  * march, four Allen-Cahn or two Cahn-Hilliard steps per pass on 26 x 52, 32 x
- * 32, 16 x 32 and 16 x 16 tiles, in the FP64 form also 16 x 64, in FP32 32 x 64
+ * 32, 16 x 32, 16 x 16 and 26 x 56 tiles, in the FP64 form also 16 x 64, in
+ * FP32 32 x 64 and 30 x 56
  * (their default where it is the fastest; a default reports the body of the
  * pass it stands for, 7 for Cahn-Hilliard and 12 or 8 for Allen-Cahn). 2-D periodic grain growth
  * and Zener pinning with 2, 4, 8, 16 or 32 fields in the same forms: 16 is the

@@ -475,9 +475,10 @@ int mmspx_set_tile(mmspx_state* s, int ty, int tz, int chunk)
 	if (s->geom.dim == 3 && ty == 32 && tz == 32) opt = 7;
 	else if (s->geom.dim == 3 && s->tuned && s->tile.opt == 6 && ty == 32 && tz == 64) opt = 6;
 	else if (s->geom.dim == 3 && s->tuned && (s->tile.opt == 8 || s->tile.opt == 12)) opt = s->tile.opt;
-	// 26 x 52 and 16 x 16 name the 3-D four-level march
+	// 26 x 52, 16 x 16 and the tiles of 56 columns name the 3-D four-level march
 	if (s->geom.dim == 3 && ((s->tuned && s->tile.opt == 15 && march4_tile_known(s->desc.precision, ty, tz)) ||
-	                         (ty == 26 && tz == 52) || (ty == 16 && tz == 16)))
+	                         (ty == 26 && tz == 52) || (ty == 16 && tz == 16) ||
+	                         (tz == 56 && march4_tile_known(s->desc.precision, ty, tz))))
 		opt = 15;
 	TuneChoice t{2, ty, tz, chunk, opt};
 	if (!tile_known(s->geom, t)) return fail(MMSPX_EINVAL, "no compiled tile of that shape for this grid");

@@ -16,9 +16,10 @@
 // a row takes two barriers however many waves and levels there are, and one
 // LDS read per square. With one wave (W = 1) the sums stay in registers.
 //
-// Bound by vector instructions (about 18 per field, node and step, which fill
-// 95 % of the issue slots at 2048^2 x 32 FP32: 82.5 us per step, where moving
-// the grid once per four steps takes 60). Two fields per wave, so that many
+// A four-step pass over 2048^2 x 32 FP32 takes 330 us, of which moving the grid
+// once takes 240 and vector work (about 18 instructions per field, node and
+// step at 2.3 cycles, 4.4 where a shift is folded in) about 200 beside it, on
+// 64/56 of the columns. Two fields per wave, so that many
 // waves meet the latencies of a row: 2048^2 x 32 FP32 85.4 us with four,
 // 512^2 x 8 FP32 4.3 against 3.6; four where one wave then holds all of them
 // and needs no exchange (2048^2 x 4 FP32 11.4 us, 12.4 on two waves).

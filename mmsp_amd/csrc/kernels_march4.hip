@@ -22,13 +22,14 @@ bool march4_supported(const Geom& g, int prec, int model)
 
 int march4_max_steps(int model) { return model == MMSPX_AC ? 4 : 2; }
 
-static const int kTiles[2][5][2] = {{{26, 52}, {16, 64}, {32, 32}, {16, 32}, {16, 16}},
-                                    {{32, 64}, {26, 52}, {32, 32}, {16, 32}, {16, 16}}};
+// the last two have a wave's lanes along axis 2 (wmarch4.hpp)
+static const int kTiles[2][7][2] = {{{26, 52}, {16, 64}, {32, 32}, {16, 32}, {16, 16}, {26, 56}, {0, 0}},
+                                    {{32, 64}, {26, 52}, {32, 32}, {16, 32}, {16, 16}, {26, 56}, {30, 56}}};
 
 bool march4_tile_known(int prec, int ty, int tz)
 {
 	for (auto& t : kTiles[prec == MMSPX_F64 ? 0 : 1])
-		if (t[0] == ty && t[1] == tz) return true;
+		if (ty > 0 && t[0] == ty && t[1] == tz) return true;
 	return false;
 }
 
@@ -36,17 +37,19 @@ bool march4_tile_known(int prec, int ty, int tz)
 // c + 6 iterations (the march starts three planes early and ends three late);
 // tau is the time of one iteration when 1, 2, .. workgroups share a CU
 // (microseconds, Cahn-Hilliard; the last entry is how many fit), a launch
-// takes full rounds of 256 CUs and one of what is left. Fitted to a sweep of
-// chunks of 3 to 64 planes on 14 grids from 32^3 to 256^3, odd ones among
-// them. Against the former defaults (us per step): Allen-Cahn FP64 64^3 4.4
-// -> 3.3, 150 x 203 x 97 17.4 -> 7.7, 256^3 31.6 -> 27.4; FP32 150 x 203 x 97
-// 12.2 -> 5.2, 256^3 19.0 -> 13.4; Cahn-Hilliard FP64 64^3 8.0 -> 5.8, 150 x
-// 203 x 97 19.3 -> 12.1, 256^3 46.4 -> 42.1; FP32 150 x 203 x 97 13.9 -> 9.9,
-// 256^3 29.1 -> 24.3. The two-step register queues on 32 x 32 tiles (body 7)
-// stay where they are faster: FP64 Cahn-Hilliard on grids that 32 x 32 tiles
-// and their chunks divide into one round (128^3 9.6 against 10.6).
+// takes full rounds of 256 CUs and one of what is left. Fitted to sweeps of
+// chunks of 3 to 64 planes on 18 grids from 32^3 to 320^3, odd ones among
+// them; it picks the best measured or within 5 % of it. Against the one- and
+// two-step marches and register queues before (us per step): Allen-Cahn FP64
+// 64^3 4.4 -> 3.3, 150 x 203 x 97 17.4 -> 6.8, 256^3 31.6 -> 23.7; FP32 150 x
+// 203 x 97 12.2 -> 4.8, 256^3 19.0 -> 13.3; Cahn-Hilliard FP64 64^3 8.0 ->
+// 5.6, 128^3 10.4 -> 9.6, 150 x 203 x 97 19.3 -> 10.6, 256^3 46.4 -> 38.6;
+// FP32 150 x 203 x 97 13.9 -> 8.0, 256^3 29.1 -> 22.3. The tiles with lanes
+// along axis 2 are the fastest from about 96^3 on; Allen-Cahn in FP32, where
+// they save least, takes them as 9 % slower (192^3 26 x 56 tiles 8.0 us, 32 x
+// 64 7.2; Cahn-Hilliard 13.0 and 13.1).
 // us of one launch: `wgs` workgroups of c + 6 iterations, ta[n-1] us each with n to a CU
-static double march_time(int64_t wgs, int c, const double (&ta)[6])
+static double march_time(int64_t wgs, int c, const double* ta)
 {
 	int cap = 0;
 	while (cap < 6 && ta[cap] > 0.0) cap++;
@@ -59,22 +62,23 @@ static int64_t march_wgs(const Geom& g, int ty, int tz, int c)
 	return (int64_t)((g.n[1] + ty - 1) / ty) * ((g.n[2] + tz - 1) / tz) * ((g.n[0] + c - 1) / c);
 }
 
-static TuneChoice march_best(const Geom* const* g, int count, int prec, double* us)
+static TuneChoice march_best(const Geom* const* g, int count, int prec, int model, int tiles)
 {
-	static const double tau[2][5][6] = {
-	    {{1.45}, {1.36}, {1.36}, {1.00, 1.51}, {0.92, 1.10, 1.30, 1.51}},
-	    {{1.31}, {1.08, 1.64}, {1.05, 1.41}, {0.79, 1.00, 1.26, 1.52}, {0.77, 0.86, 0.96, 1.06, 1.16, 1.26}}};
+	static const double tau[2][7][6] = {
+	    {{1.45}, {1.36}, {1.36}, {1.00, 1.51}, {0.92, 1.10, 1.30, 1.51}, {1.30}, {}},
+	    {{1.31}, {1.08, 1.64}, {1.05, 1.41}, {0.79, 1.00, 1.26, 1.52}, {0.77, 0.86, 0.96, 1.06, 1.16, 1.26}, {0.97, 1.39}, {1.10, 1.62}}};
 	const int f = prec == MMSPX_F64 ? 0 : 1;
 	TuneChoice out{2, 16, 32, 8, 15};
-	*us = 1e300;
-	for (int k = 0; k < 5; k++) {
+	double us = 1e300;
+	for (int k = 0; k < tiles; k++) {
 		const int ty = kTiles[f][k][0], tz = kTiles[f][k][1];
+		if (ty == 0) continue;
 		for (int c = 3; c <= 64; c += count > 1 && c >= 8 ? 4 : 1) {
 			int64_t wgs = 0;
 			for (int m = 0; m < count; m++) wgs += march_wgs(*g[m], ty, tz, c);
-			const double t = march_time(wgs, c, tau[f][k]);
-			if (t < *us) {
-				*us = t;
+			const double t = march_time(wgs, c, tau[f][k]) * (k >= 5 && f == 1 && model == MMSPX_AC ? 1.09 : 1.0);
+			if (t < us) {
+				us = t;
 				out = TuneChoice{2, ty, tz, c, 15};
 			}
 		}
@@ -84,21 +88,14 @@ static TuneChoice march_best(const Geom* const* g, int count, int prec, double* 
 
 TuneChoice march4_choice_many(const Geom* const* g, int count, int prec)
 {
-	double us;
-	return march_best(g, count, prec, &us);
+	return march_best(g, count, prec, MMSPX_CH, 5);  // the tiles the batch kernels are built for
 }
 
 bool march4_choice(const Geom& g, int prec, int model, TuneChoice* out)
 {
 	if (!march4_supported(g, prec, model)) return false;
 	const Geom* one = &g;
-	double us;
-	*out = march_best(&one, 1, prec, &us);
-	if (prec == MMSPX_F64 && model != MMSPX_AC) {
-		static const double queues[6] = {1.25};
-		for (int c : {6, 8, 12, 16, 24, 32, 48, 64})
-			if (march_time(march_wgs(g, 32, 32, c), c, queues) < us) return false;
-	}
+	*out = march_best(&one, 1, prec, model, 7);
 	return true;
 }
 

@@ -4,7 +4,7 @@
 
 #include <type_traits>
 
-#include "march4.hpp"
+#include "wmarch4.hpp"
 
 namespace mmspx {
 
@@ -37,6 +37,36 @@ static int launch_march4_body(const Geom& g, const ModelParams& p, const void* a
 	return 0;
 }
 
+template <int PREC, int MODEL, int NW, int R, int LEVELS, bool UNIT>
+__global__ void __launch_bounds__(64 * NW) wmarch4_k(const typename Form<PREC>::S* __restrict__ a,
+                                                     typename Form<PREC>::S* __restrict__ b, Geom g, ModelParams p,
+                                                     int chunk_len, int tiles_y, int tiles_z, int ntiles)
+{
+	int tile = blockIdx.x;
+	if ((gridDim.x & 7) == 0) tile = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+	if (tile >= ntiles) return;
+	const int tz = tile % tiles_z;
+	const int t2 = tile / tiles_z;
+	const int ty = t2 % tiles_y;
+	const int xb = t2 / tiles_y * chunk_len;
+	wmarch4<PREC, MODEL, NW, R, LEVELS, UNIT>(a, b, g, p, ty * (NW * R - 6), tz * 56, xb, min(xb + chunk_len, g.n[0]));
+}
+
+template <int PREC, int MODEL, int NW, int R, int LEVELS, bool UNIT>
+static int launch_wmarch4_body(const Geom& g, const ModelParams& p, const void* a, void* b, hipStream_t st, int chunk)
+{
+	using S = typename Form<PREC>::S;
+	constexpr int TY = NW * R - 6, TZ = 56;
+	const int tiles_y = (g.n[1] + TY - 1) / TY;
+	const int tiles_z = (g.n[2] + TZ - 1) / TZ;
+	const int ntiles = tiles_y * tiles_z * ((g.n[0] + chunk - 1) / chunk);
+	// a last pass of fewer steps multiplies by unit weights too
+	hipLaunchKernelGGL((wmarch4_k<PREC, MODEL, NW, R, LEVELS, UNIT && LEVELS == 4>), dim3((ntiles + 7) / 8 * 8),
+	                   dim3(64 * NW), 0, st, (const S*)a, (S*)b, g, p, chunk, tiles_y, tiles_z, ntiles);
+	MMSPX_HIP(hipGetLastError());
+	return 0;
+}
+
 template <int PREC, int MODEL, int LEVELS, bool UNIT>
 static int launch_march4_tile(const Geom& g, const ModelParams& p, const void* a, void* b, hipStream_t st,
                               const TuneChoice& t)
@@ -45,6 +75,11 @@ static int launch_march4_tile(const Geom& g, const ModelParams& p, const void* a
 	if (t.ty == 32 && t.tz == 32) return launch_march4_body<PREC, MODEL, 32, 32, 384, LEVELS, UNIT>(g, p, a, b, st, t.chunk);
 	if (t.ty == 16 && t.tz == 32) return launch_march4_body<PREC, MODEL, 16, 32, 256, LEVELS, UNIT>(g, p, a, b, st, t.chunk);
 	if (t.ty == 16 && t.tz == 16) return launch_march4_body<PREC, MODEL, 16, 16, 128, LEVELS, UNIT>(g, p, a, b, st, t.chunk);
+	// a wave's lanes along axis 2
+	if (t.ty == 26 && t.tz == 56) return launch_wmarch4_body<PREC, MODEL, 16, 2, LEVELS, UNIT>(g, p, a, b, st, t.chunk);
+	if constexpr (PREC == MMSPX_F32) {
+		if (t.ty == 30 && t.tz == 56) return launch_wmarch4_body<PREC, MODEL, 12, 3, LEVELS, UNIT>(g, p, a, b, st, t.chunk);
+	}
 	// a wide tile: 16 x 64 in double (the registers of 32 x 64 do not fit), 32 x 64 in float
 	if constexpr (PREC == MMSPX_F64) {
 		if (t.ty == 16 && t.tz == 64) return launch_march4_body<PREC, MODEL, 16, 64, 448, LEVELS, UNIT>(g, p, a, b, st, t.chunk);
