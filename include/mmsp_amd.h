@@ -283,18 +283,23 @@ int mmspx_set_tile(mmspx_state* s, int ty, int tz, int chunk);
  * registers (their default). 3-D periodic Allen-Cahn and Cahn-Hilliard
  * (deterministic chemical potentials) in the same forms: 15 is the four-level
  * march, four Allen-Cahn or two Cahn-Hilliard steps per pass on 26 x 52, 32 x
- * 32, 16 x 32, 16 x 16 and 26 x 56 tiles, in the FP64 form also 16 x 64, in
- * FP32 32 x 64 and 30 x 56
+ * 32, 16 x 32, 16 x 16 and 26 x 56 tiles, in the FP64 form also 16 x 64
+ * and 42 x 56, in FP32 32 x 64 and 30 x 56
  * (their default where it is the fastest; a default reports the body of the
  * pass it stands for, 7 for Cahn-Hilliard and 12 or 8 for Allen-Cahn). 2-D periodic grain growth
  * and Zener pinning with 2, 4, 8, 16 or 32 fields in the same forms: 16 is the
- * four-step field strips, 1 x 56 tiles (their default). */
+ * four-step field strips, 1 x 56 tiles (their default). 3-D periodic grain
+ * growth and Zener pinning with 2, 4 or 8 fields in the same forms: 17 is the
+ * field march, two to four steps per pass on tiles of 60, 58 or 56 columns
+ * (their default where it is the fastest; a default reports the body it stands
+ * for, 12 or 8). */
 int mmspx_set_tile_options(mmspx_state* s, int body);
 /* Returns variant + 16 * tile body (1: register queues, or the 2-D
  * grain-growth tile; 2: wave strips, or 3-D register queues on 768 threads;
  * 3: temporal blocks, or 3-D register queues on 1024 threads; 4 and 5: the
  * split strips on two and four waves; 13 and 14: the multi-step wave strips; 15: the
- * 3-D four-level march; 16: the four-step field strips). Before any tile is
+ * 3-D four-level march; 16: the four-step field strips; 17: the 3-D field
+ * march). Before any tile is
  * set, reports what the last step ran (the Cahn-Hilliard default before any step). */
 int mmspx_get_tile(const mmspx_state* s, int* ty, int* tz, int* chunk);
 /* Project autotuner: times every candidate tile for `model` on this state's

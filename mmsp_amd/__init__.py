@@ -326,7 +326,7 @@ class Grid:
         14 the 2-D multi-step wave strips of Allen-Cahn and Cahn-Hilliard
         (eight or four levels of the update per pass); 15 their 3-D four-level
         march (periodic); 16 the four-step field strips of 2-D grain growth and
-        Zener pinning (periodic)."""
+        Zener pinning and 17 their 3-D field march (periodic)."""
         check(lib.mmspx_set_tile_options(self._h, int(body) if body is not None else (1 if register_queues else 0)))
 
     def get_tile(self):

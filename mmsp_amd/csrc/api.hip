@@ -378,6 +378,7 @@ static int step_impl(mmspx_state* s, int model, const double* params, int np, in
 	}
 	s->last = fused ? tc : TuneChoice{1, 0, 0, 0, 0};
 	if (s->last.opt == 15) s->last.opt = march4_reported_body(g, model);
+	if (s->last.opt == 17) s->last.opt = one_step_choice(g, s->desc.precision, model).opt;
 	s->has_last = true;
 	const int spl = fused ? fused_steps_per_launch(model, tc) : 1;
 	if ((((ch_family(model) || model == MMSPX_OSTWALD) && !fused) || (fused && fused_needs_plane(g, model, tc))) &&
@@ -480,6 +481,10 @@ int mmspx_set_tile(mmspx_state* s, int ty, int tz, int chunk)
 	                         (ty == 26 && tz == 52) || (ty == 16 && tz == 16) ||
 	                         (tz == 56 && march4_tile_known(s->desc.precision, ty, tz))))
 		opt = 15;
+	// the 3-D field march keeps its body on its own tiles
+	if (s->geom.dim == 3 && s->tuned && s->tile.opt == 17 &&
+	    fmarch_tile_known(s->desc.precision, s->geom.fields, ty, tz))
+		opt = 17;
 	TuneChoice t{2, ty, tz, chunk, opt};
 	if (!tile_known(s->geom, t)) return fail(MMSPX_EINVAL, "no compiled tile of that shape for this grid");
 	s->tile = t;
@@ -490,10 +495,10 @@ int mmspx_set_tile(mmspx_state* s, int ty, int tz, int chunk)
 int mmspx_set_tile_options(mmspx_state* s, int body)
 {
 	if (!s) return fail(MMSPX_EINVAL, "null state");
-	if (body < 0 || body > 16 || (body == 3 && s->geom.dim != 3) ||
+	if (body < 0 || body > 17 || (body == 3 && s->geom.dim != 3) ||
 	    ((body == 4 || body == 5 || (body >= 9 && body <= 11) || body == 13 || body == 14 || body == 16) &&
 	     s->geom.dim != 2) ||
-	    (((body >= 6 && body <= 8) || body == 12 || body == 15) && s->geom.dim != 3))
+	    (((body >= 6 && body <= 8) || body == 12 || body == 15 || body == 17) && s->geom.dim != 3))
 		return fail(MMSPX_EINVAL, "unknown tile body");
 	if (!s->tuned) {
 		s->tile = one_step_choice(s->geom, s->desc.precision, MMSPX_CH_DW);
@@ -519,7 +524,13 @@ int mmspx_set_tile_options(mmspx_state* s, int body)
 	// two-step march 16 x 32 for every model)
 	if (s->geom.dim == 3 && s->tile.variant == 2) {
 		const int ty = s->tile.ty, tz = s->tile.tz;
-		if (body == 15) {
+		if (body == 17) {
+			if (!fmarch_tile_known(s->desc.precision, s->geom.fields, ty, tz)) {
+				const TuneChoice any = fmarch_any_tile(s->desc.precision, s->geom.fields, s->tile.chunk);
+				s->tile.ty = any.ty;
+				s->tile.tz = any.tz;
+			}
+		} else if (body == 15) {
 			if (!march4_tile_known(s->desc.precision, ty, tz)) {
 				s->tile.ty = 16;
 				s->tile.tz = 32;

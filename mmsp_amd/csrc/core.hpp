@@ -177,6 +177,16 @@ TuneChoice march4_choice_many(const Geom* const* g, int count, int prec);  // on
 int march4_reported_body(const Geom& g, int model);
 int launch_march4(const Geom& g, int prec, const ModelParams& p, const void* a, void* b, hipStream_t st,
                   const TuneChoice& t, int nsteps);
+// 3-D field march (kernels_fmarch.hip), tile body 17: grain growth and Zener
+// pinning, several steps per pass (fmarch_steps of its tile)
+bool fmarch_supported(const Geom& g, int prec, int model);
+bool fmarch_tile_known(int prec, int fields, int ty, int tz);
+TuneChoice fmarch_any_tile(int prec, int fields, int chunk);
+inline int fmarch_steps(const TuneChoice& t) { return (64 - t.tz) / 2; }
+bool fmarch_choice(const Geom& g, int prec, int model, TuneChoice* out);
+int fmarch_candidates(const Geom& g, int prec, int model, TuneChoice* out, int max);
+int launch_fmarch(const Geom& g, int prec, const ModelParams& p, const void* a, void* b, hipStream_t st,
+                  const TuneChoice& t, int nsteps);
 // 2-D four-step field strips (kernels_fields2d.hip), tile body 16: grain growth
 // and Zener pinning, strips of kSteps4Cols columns, `chunk` rows per workgroup
 constexpr int kFieldsSteps = 4;

@@ -387,6 +387,7 @@ TuneChoice default_choice(const Geom& g, int prec, int model)
 	TuneChoice t;
 	if (steps2d_choice(g, prec, model, &t)) return t;
 	if (fields2d_choice(g, prec, model, &t)) return t;
+	if (fmarch_choice(g, prec, model, &t)) return t;
 	if (march4_choice(g, prec, model, &t)) return t;
 	return one_step_choice(g, prec, model);
 }
@@ -555,6 +556,8 @@ TuneChoice one_step_choice(const Geom& g, int prec, int model)
 bool tile_known(const Geom& g, const TuneChoice& t)
 {
 	if (t.chunk < 2 || t.chunk > 4096) return false;
+	if (g.dim == 3 && t.opt == 17)
+		return fmarch_tile_known(MMSPX_F64, g.fields, t.ty, t.tz) || fmarch_tile_known(MMSPX_F32, g.fields, t.ty, t.tz);
 	if (g.dim == 3 && t.opt == 15)
 		return march4_tile_known(MMSPX_F64, t.ty, t.tz) || march4_tile_known(MMSPX_F32, t.ty, t.tz);
 	if (g.dim == 3)
@@ -577,7 +580,8 @@ int tile_candidates(const Geom& g, int prec, int model, TuneChoice* out, int max
 		if (n < max) out[n++] = TuneChoice{2, ty, tz, chunk, opt};
 	};
 	const bool ch = ch_family(model);
-	// grain growth and Zener pinning, periodic: four steps per pass
+	// grain growth and Zener pinning, periodic: several steps per pass
+	n += fmarch_candidates(g, prec, model, out + n, max - n);
 	if (fields2d_supported(g, prec, model))
 		for (int c : {8, 16, 32, 64, 128}) add(1, kSteps4Cols, c, 16);
 	if (g.dim == 2 && model == MMSPX_OSTWALD) {
@@ -1283,6 +1287,7 @@ static int launch_prec(const Geom& g, const ModelParams& p, const void* a, void*
 	const int chunk = t.chunk > 0 ? t.chunk : 32;
 	if (g.dim == 2 && (t.opt == 13 || t.opt == 14)) return launch_steps2d(g, PREC, p, a, b, st, t.opt, chunk, nsteps);
 	if (g.dim == 2 && t.opt == 16) return launch_fields2d(g, PREC, p, a, b, st, chunk, nsteps);
+	if (g.dim == 3 && t.opt == 17) return launch_fmarch(g, PREC, p, a, b, st, t, nsteps);
 	if (g.dim == 3 && t.opt == 15) return launch_march4(g, PREC, p, a, b, st, t, nsteps);
 	switch (p.model) {
 	case MMSPX_CH: return launch_ch_prec<PREC, 0>(g, p, a, b, st, t, nsteps);
@@ -1361,6 +1366,7 @@ int fused_steps_per_launch(int model, const TuneChoice& t)
 		return steps2d_max_steps(model, t.opt);
 	if ((model == MMSPX_AC || model == MMSPX_CH || model == MMSPX_CH_DW) && t.opt == 15) return march4_max_steps(model);
 	if ((model == MMSPX_GG || model == MMSPX_ZENER) && t.opt == 16) return kFieldsSteps;
+	if ((model == MMSPX_GG || model == MMSPX_ZENER) && t.opt == 17) return fmarch_steps(t);
 	if (model == MMSPX_AC && t.tz == kTbCols) return std::max(1, std::min(t.chunk, kTbMaxSteps));
 	if ((model == MMSPX_CH || model == MMSPX_CH_DW) && (t.opt == 6 || t.opt == 7)) return 2;
 	if ((model == MMSPX_GG || model == MMSPX_ZENER) && t.opt >= 9 && t.opt <= 11) return 2;

@@ -23,13 +23,13 @@ bool march4_supported(const Geom& g, int prec, int model)
 int march4_max_steps(int model) { return model == MMSPX_AC ? 4 : 2; }
 
 // the last two have a wave's lanes along axis 2 (wmarch4.hpp)
-static const int kTiles[2][7][2] = {{{26, 52}, {16, 64}, {32, 32}, {16, 32}, {16, 16}, {26, 56}, {0, 0}},
+static const int kTiles[2][7][2] = {{{26, 52}, {16, 64}, {32, 32}, {16, 32}, {16, 16}, {26, 56}, {42, 56}},
                                     {{32, 64}, {26, 52}, {32, 32}, {16, 32}, {16, 16}, {26, 56}, {30, 56}}};
 
 bool march4_tile_known(int prec, int ty, int tz)
 {
 	for (auto& t : kTiles[prec == MMSPX_F64 ? 0 : 1])
-		if (ty > 0 && t[0] == ty && t[1] == tz) return true;
+		if (t[0] == ty && t[1] == tz) return true;
 	return false;
 }
 
@@ -65,14 +65,13 @@ static int64_t march_wgs(const Geom& g, int ty, int tz, int c)
 static TuneChoice march_best(const Geom* const* g, int count, int prec, int model, int tiles)
 {
 	static const double tau[2][7][6] = {
-	    {{1.45}, {1.36}, {1.36}, {1.00, 1.51}, {0.92, 1.10, 1.30, 1.51}, {1.30}, {}},
+	    {{1.45}, {1.36}, {1.36}, {1.00, 1.51}, {0.92, 1.10, 1.30, 1.51}, {1.30}, {1.94}},
 	    {{1.31}, {1.08, 1.64}, {1.05, 1.41}, {0.79, 1.00, 1.26, 1.52}, {0.77, 0.86, 0.96, 1.06, 1.16, 1.26}, {0.97, 1.39}, {1.10, 1.62}}};
 	const int f = prec == MMSPX_F64 ? 0 : 1;
 	TuneChoice out{2, 16, 32, 8, 15};
 	double us = 1e300;
 	for (int k = 0; k < tiles; k++) {
 		const int ty = kTiles[f][k][0], tz = kTiles[f][k][1];
-		if (ty == 0) continue;
 		for (int c = 3; c <= 64; c += count > 1 && c >= 8 ? 4 : 1) {
 			int64_t wgs = 0;
 			for (int m = 0; m < count; m++) wgs += march_wgs(*g[m], ty, tz, c);

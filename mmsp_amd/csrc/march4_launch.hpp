@@ -77,7 +77,9 @@ static int launch_march4_tile(const Geom& g, const ModelParams& p, const void* a
 	if (t.ty == 16 && t.tz == 16) return launch_march4_body<PREC, MODEL, 16, 16, 128, LEVELS, UNIT>(g, p, a, b, st, t.chunk);
 	// a wave's lanes along axis 2
 	if (t.ty == 26 && t.tz == 56) return launch_wmarch4_body<PREC, MODEL, 16, 2, LEVELS, UNIT>(g, p, a, b, st, t.chunk);
-	if constexpr (PREC == MMSPX_F32) {
+	if constexpr (PREC == MMSPX_F64) {
+		if (t.ty == 42 && t.tz == 56) return launch_wmarch4_body<PREC, MODEL, 12, 4, LEVELS, UNIT>(g, p, a, b, st, t.chunk);
+	} else {
 		if (t.ty == 30 && t.tz == 56) return launch_wmarch4_body<PREC, MODEL, 12, 3, LEVELS, UNIT>(g, p, a, b, st, t.chunk);
 	}
 	// a wide tile: 16 x 64 in double (the registers of 32 x 64 do not fit), 32 x 64 in float

@@ -48,6 +48,37 @@ __device__ __forceinline__ double shift_next(double v)
 	return __builtin_bit_cast(double, make_int2(shift_next(s.x), shift_next(s.y)));
 }
 
+// Keeps a store's value computed where it stands (not moved under the store's
+// condition, which would split the march into a branch per row and the lane
+// shifts from the arithmetic they fold into).
+template <typename T>
+__device__ __forceinline__ void keep_value(T& v)
+{
+	asm volatile("" : "+v"(v));
+}
+// A row's start, the same for every lane, in scalar registers: accesses at a
+// lane's byte offset from it take the offset from one vector register (and not a
+// 64-bit vector sum per row, some of them kept through the march).
+template <typename T>
+using GlobalT = __attribute__((address_space(1))) T;
+template <typename T>
+__device__ __forceinline__ GlobalT<T>* scalar_row(T* p)
+{
+	GlobalT<T>* q = (GlobalT<T>*)p;
+	asm volatile("" : "+s"(q));
+	return q;
+}
+template <typename T>
+__device__ __forceinline__ T load_at(const T* row, unsigned byte)
+{
+	return *(const GlobalT<T>*)((const GlobalT<char>*)scalar_row(row) + byte);
+}
+template <typename T>
+__device__ __forceinline__ void store_at(T* row, unsigned byte, T v)
+{
+	*(GlobalT<T>*)((GlobalT<char>*)scalar_row(row) + byte) = v;
+}
+
 enum { S2_AC = 0, S2_CH = 1, S2_CH_DW = 2 };
 
 // The two-axis laplacian of y in the reference's order. yh - 2y is one fma:

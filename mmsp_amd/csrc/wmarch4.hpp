@@ -15,7 +15,8 @@
 // Cahn-Hilliard 42 us per step: 22 and 20). Here vector work is 73 % of the
 // time at the rates the instructions reach (4.3 cycles for a double add or a
 // shift), the rest waits at the barrier; 16 waves of two rows, the most a
-// workgroup holds: 256^3 FP64 Cahn-Hilliard 35.7 us per step, Allen-Cahn 24.4
+// workgroup holds, or 12 of four where the grid gives each enough planes (320^3
+// 67 against 84 us): 256^3 FP64 Cahn-Hilliard 35.7 us per step, Allen-Cahn 24.4
 // (8 waves of four rows 38.3 and 25.6; a column pair per lane, which halves
 // the shifts, 40.1 and 26.4; levels two planes apart instead of one, so that
 // none waits for another, 37.3 and 25.4).
@@ -65,21 +66,23 @@ __device__ __forceinline__ void wmarch4(const typename Form<PREC>::S* __restrict
 	const int lane = threadIdx.x & 63;
 	const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
 	const int z = z0 - 4 + lane;
-	const unsigned zc = (unsigned)wrap(z, nz);
+	// a row's address is scalar, the lane's byte offset in it 32 bits
+	const unsigned zc = (unsigned)wrap(z, nz) * (unsigned)sizeof(S);
+	auto uniform = [](int v) { return (unsigned)__builtin_amdgcn_readfirstlane(v); };
 	const bool zout = lane >= 4 && lane < 60 && z < nz;
 	// the wave's rows of the tile and its three-row halo, wave-uniform
 	const int r0 = wv * R;
 	unsigned row[R];
-	bool out[R];
 #pragma unroll
 	for (int k = 0; k < R; k++) {
 		const int r = r0 + k, y = y0 - 3 + r;
-		row[k] = (unsigned)wrap(y, ny) * (unsigned)nz;
-		out[k] = r >= 3 && r < TY + 3 && y < ny;
+		row[k] = uniform(wrap(y, ny)) * (unsigned)nz;
 	}
+	// the rows that are written: 3 <= r < TY + 3 and y < ny
+	const int klo = 3 - r0, khi = min(TY + 3, ny - y0 + 3) - r0;
 	const bool first = wv == 0, last = wv == NW - 1;
-	const unsigned rrow = (unsigned)wrap(first ? y0 - 4 : y0 + TY + 3, ny) * (unsigned)nz;
-	int wx = wrap(xb - 4, nx);
+	const unsigned rrow = uniform(wrap(first ? y0 - 4 : y0 + TY + 3, ny)) * (unsigned)nz;
+	int wx = (int)uniform(wrap(xb - 4, nx));
 	auto src_next = [&]() {
 		const S* s = a + (int64_t)wx * plane;
 		wx = wx + 1 == nx ? 0 : wx + 1;
@@ -94,13 +97,14 @@ __device__ __forceinline__ void wmarch4(const typename Form<PREC>::S* __restrict
 	for (int k = 0; k < R; k++)
 #pragma unroll
 		for (int s = 0; s < 3; s++) v1[s][k] = v2[s][k] = v3[s][k] = 0;
+	unsigned o = zc;
 	const S* ring_src = nullptr;
 #pragma unroll
 	for (int s = 0; s < 3; s++) {
 		ring_src = src_next();
 #pragma unroll
-		for (int k = 0; k < R; k++) f[s][k] = (ring_src + row[k])[zc];
-		if (s == 1 && (first || last)) rg[0] = (ring_src + rrow)[zc];
+		for (int k = 0; k < R; k++) f[s][k] = load_at(ring_src + row[k], o);
+		if (s == 1 && (first || last)) rg[0] = load_at(ring_src + rrow, o);
 	}
 
 	auto publish = [&](int level, int buf, const S (&v)[R]) {
@@ -142,11 +146,15 @@ __device__ __forceinline__ void wmarch4(const typename Form<PREC>::S* __restrict
 		S(&fm)[R] = f[j % 3];
 		S(&fc)[R] = f[(j + 1) % 3];
 		S(&fp)[R] = f[(j + 2) % 3];
-		if (first || last) rg[(j + 1) & 1] = (ring_src + rrow)[zc];
+		if (first || last) {
+			keep_value(o);
+			rg[(j + 1) & 1] = load_at(ring_src + rrow, o);
+		}
 		auto load = [&]() {
 			ring_src = src_next();
+			keep_value(o);
 #pragma unroll
-			for (int k = 0; k < R; k++) fm[k] = (ring_src + row[k])[zc];
+			for (int k = 0; k < R; k++) fm[k] = load_at(ring_src + row[k], o);
 		};
 		const int w = j & 1, r = w ^ 1;
 		publish(0, w, fc);
@@ -161,7 +169,12 @@ __device__ __forceinline__ void wmarch4(const typename Form<PREC>::S* __restrict
 		// the written level's row k, at plane x
 		auto write = [&](int x, int k, S v) {
 			if (LEVELS < 4 && (x < xb || x >= xe)) return;
-			if (out[k] && zout) (b + (int64_t)x * plane + row[k])[zc] = v;
+			keep_value(v);
+			if (k >= klo && k < khi)
+				if (zout) {
+					keep_value(o);
+					store_at(b + (int64_t)x * plane + row[k], o, v);
+				}
 		};
 		S(&a1)[R] = v1[j % 3];
 		S(&b1)[R] = v1[(j + 2) % 3];  // P-1
