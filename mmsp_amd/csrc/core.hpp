@@ -177,6 +177,8 @@ TuneChoice march4_choice_many(const Geom* const* g, int count, int prec);  // on
 int march4_reported_body(const Geom& g, int model);
 int launch_march4(const Geom& g, int prec, const ModelParams& p, const void* a, void* b, hipStream_t st,
                   const TuneChoice& t, int nsteps);
+// 2-D multi-phase grain growth, wave strips (kernels_gga2d.hip)
+int launch_gga2d(const Geom& g, int prec, const ModelParams& p, const void* a, void* b, hipStream_t st, int chunk);
 // 3-D field march (kernels_fmarch.hip), tile body 17: grain growth and Zener
 // pinning, several steps per pass (fmarch_steps of its tile)
 bool fmarch_supported(const Geom& g, int prec, int model);

@@ -465,6 +465,79 @@ __device__ __forceinline__ void gga_rates(const typename Form<PREC>::S (&phi)[QM
 	}
 }
 
+// gga_rates over the first n (2 to 4) of 4 slots, the same additions in the same
+// order: a field's term c2*lap + w*phi and 3*phi are formed once, and the second
+// rate of a pair subtracts the negative of the first's, so it adds it (dF[j] -
+// dF[h] is exactly -(dF[h] - dF[j]), and a rate that starts at +0 is never -0).
+template <int PREC>
+__device__ __forceinline__ void gga_rates4(const typename Form<PREC>::S (&phi)[4], const typename Form<PREC>::S (&lap)[4],
+                                           int n, const ModelParams& p, typename Form<PREC>::S (&dp)[4])
+{
+	using S = typename Form<PREC>::S;
+	constexpr bool dbl = PREC == MMSPX_F64;
+	const S c2 = dbl ? (S)p.an[AN_C2] : (S)p.anf[AN_C2];
+	const S w = dbl ? (S)p.an[AN_W] : (S)p.anf[AN_W];
+	const S mu = dbl ? (S)p.an[AN_MU] : (S)p.anf[AN_MU];
+	S dF[4], e[4], t[4];
+#pragma unroll
+	for (int h = 0; h < 4; h++) {
+		e[h] = c2 * lap[h] + w * phi[h];
+		t[h] = S(3) * phi[h];
+		dF[h] = 0;
+		dp[h] = 0;
+	}
+#pragma unroll
+	for (int h = 0; h < 4; h++)
+#pragma unroll
+		for (int j = h + 1; j < 4; j++)
+			if (j < n) {
+				dF[h] += e[j];
+				dF[j] += e[h];
+#pragma unroll
+				for (int k = j + 1; k < 4; k++)
+					if (k < n) {
+						dF[h] += t[j] * phi[k];
+						dF[j] += t[k] * phi[h];
+						dF[k] += t[h] * phi[j];
+					}
+			}
+#pragma unroll
+	for (int h = 0; h < 4; h++)
+#pragma unroll
+		for (int j = h + 1; j < 4; j++)
+			if (j < n) {
+				const S m = mu * (dF[h] - dF[j]);
+				dp[h] -= m;
+				dp[j] += m;
+			}
+}
+
+// The clamped update and projection onto the simplex (graingrowth.cpp:170-185)
+// of a node with cnt fields present and rates dp; fields at or past Q are skipped.
+template <int PREC, int QMAX>
+__device__ __forceinline__ void gga_project(typename Form<PREC>::S (&phi)[QMAX], const typename Form<PREC>::S (&dp)[QMAX],
+                                            typename Form<PREC>::S cnt, int Q, const ModelParams& p)
+{
+	using S = typename Form<PREC>::S;
+	constexpr int UN = QMAX <= 8 ? QMAX : 1;
+	const S dt = PREC == MMSPX_F64 ? (S)p.an[AN_DT] : (S)p.anf[AN_DT];
+	S sum = 0;
+	const S rate = dt * (S(2) / cnt);
+#pragma unroll UN
+	for (int h = 0; h < QMAX; h++) {
+		if (h >= Q) continue;
+		S v = phi[h] + rate * dp[h];
+		if (v > S(1)) v = S(1);
+		if (v < S(0)) v = S(0);
+		phi[h] = v;
+		sum += v;
+	}
+	const S rsum = fabs(sum) > S(0) ? S(1) / sum : S(0);
+#pragma unroll UN
+	for (int h = 0; h < QMAX; h++)
+		if (h < Q) phi[h] = phi[h] * rsum;
+}
+
 // Multi-phase grain growth at one node with at least two fields present
 // (graingrowth.cpp:141-185): `act` holds the present fields (cnt of them) and
 // lap their laplacians. gga_rates, then the clamped update and the projection
@@ -478,10 +551,7 @@ __device__ __forceinline__ void gga_node(typename Form<PREC>::S (&phi)[QMAX], co
                                          uint32_t act, typename Form<PREC>::S cnt, int Q, const ModelParams& p)
 {
 	using S = typename Form<PREC>::S;
-	constexpr bool dbl = PREC == MMSPX_F64;
-	constexpr int UN = QMAX <= 8 ? QMAX : 1;
 	constexpr int K = 4;
-	const S dt = dbl ? (S)p.an[AN_DT] : (S)p.anf[AN_DT];
 	S dp[QMAX];
 	if constexpr (QMAX > K && QMAX <= 8) {
 		if (cnt <= S(K)) {
@@ -500,7 +570,7 @@ __device__ __forceinline__ void gga_node(typename Form<PREC>::S (&phi)[QMAX], co
 					}
 				}
 			}
-			gga_rates<PREC, K>(cphi, clap, (1u << (int)cnt) - 1u, p, cdp);
+			gga_rates4<PREC>(cphi, clap, (int)cnt, p, cdp);
 #pragma unroll
 			for (int f = 0; f < QMAX; f++) {
 				const bool on = act >> f & 1u;
@@ -517,22 +587,7 @@ __device__ __forceinline__ void gga_node(typename Form<PREC>::S (&phi)[QMAX], co
 	} else {
 		gga_rates<PREC, QMAX>(phi, lap, act, p, dp);
 	}
-	// clamped update and projection onto the simplex (:170-185)
-	S sum = 0;
-	const S rate = dt * (S(2) / cnt);
-#pragma unroll UN
-	for (int h = 0; h < QMAX; h++) {
-		if (h >= Q) continue;
-		S v = phi[h] + rate * dp[h];
-		if (v > S(1)) v = S(1);
-		if (v < S(0)) v = S(0);
-		phi[h] = v;
-		sum += v;
-	}
-	const S rsum = fabs(sum) > S(0) ? S(1) / sum : S(0);
-#pragma unroll UN
-	for (int h = 0; h < QMAX; h++)
-		if (h < Q) phi[h] = phi[h] * rsum;
+	gga_project<PREC, QMAX>(phi, dp, cnt, Q, p);
 }
 
 }  // namespace mmspx

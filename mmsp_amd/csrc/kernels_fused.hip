@@ -477,9 +477,9 @@ TuneChoice one_step_choice(const Geom& g, int prec, int model)
 		return all_periodic(g) ? TuneChoice{2, tb_rows, kTbCols, 8, 3} : TuneChoice{2, 1, kWaveCols, wave_chunk, 2};
 	if (model == MMSPX_AC_NOISE) return TuneChoice{2, 1, kWaveCols, wave_chunk, 2};
 	// multi-phase grain growth (one-hot grains, 8 fields): 2-row chunks below
-	// 2^21 nodes (1024^2 FP64 36.7 us per step against 39.1 with 4 rows, 40.0
-	// with 8 and 77.3 for one thread per node), 8 rows above (2048^2 FP64 139
-	// us, FP32 70; 4096^2 FP64 500, FP32 265: within 2 % of the best of 2..16)
+	// 2^21 nodes (1024^2 FP64 28.5 us per step against 32.0 with 4 rows, 33.3
+	// with 8 and 77.3 for one thread per node; 512^2 12.2, 13.7 and 17.6), 8
+	// rows above (2048^2 FP64 132 us, FP32 53.4: within 6 % of the best of 2..16)
 	if (model == MMSPX_GG_ANISO) return TuneChoice{2, 1, kWaveCols, nodes < ((int64_t)1 << 21) ? 2 : 8, 2};
 	// Ostwald ripening (4 fields): with the row rings, 4-row chunks below 2^21
 	// nodes (1024^2 FP64 17.0 us per step against 18.0 with 8 rows; the
@@ -1112,16 +1112,7 @@ static int launch_wave(const Geom& g, const ModelParams& p, const void* a, void*
 	constexpr bool wide = sizeof(typename Form<PREC>::S) == 4;
 	if (p.model == MMSPX_AC) return launch_wave_q<PREC, 1, 0>(g, p, a, b, st, chunk);
 	if (p.model == MMSPX_AC_NOISE) return launch_wave_q<PREC, 1, 2>(g, p, a, b, st, chunk);
-	if (p.model == MMSPX_GG_ANISO) {
-		if constexpr (PREC != MMSPX_F32REF) {
-			switch (g.fields) {
-			case 2: return launch_wave_q<PREC, 2, 4>(g, p, a, b, st, chunk);
-			case 4: return launch_wave_q<PREC, 4, 4>(g, p, a, b, st, chunk);
-			case 8: return launch_wave_q<PREC, 8, 4>(g, p, a, b, st, chunk);
-			}
-		}
-		return fail(MMSPX_EUNSUPPORTED, "multi-phase wave strips take 2, 4 or 8 fields in the MMSPX_F64 and MMSPX_F32 forms");
-	}
+	if (p.model == MMSPX_GG_ANISO) return launch_gga2d(g, PREC, p, a, b, st, chunk);
 	if (p.model == MMSPX_ZENER) {
 		if constexpr (PREC != MMSPX_F32REF) {
 			switch (g.fields) {

@@ -1733,10 +1733,7 @@ __device__ __forceinline__ void gg_tile(const typename Form<PREC>::S* __restrict
 // formed in the reference's order before the field updates
 // (graingrowth.cpp:91-107); KIND 0, Allen-Cahn (Q = 1, allen-cahn.cpp:68-71);
 // KIND 2, model A (Allen-Cahn plus noise, model_A.cpp:97-101); KIND 3, Zener
-// pinning (grain growth with field 0 held, zener.cpp:117-135); KIND 4,
-// multi-phase grain growth (grain_growth/anisotropic/phase_field/
-// graingrowth.cpp:108-188: the fields present among the node and its four
-// neighbours, then gga_node; fewer than two present, the node is copied).
+// pinning (grain growth with field 0 held, zener.cpp:117-135).
 template <int PREC, int Q, int KIND>
 __device__ __forceinline__ void strip_wave(const typename Form<PREC>::S* __restrict__ a,
                                            typename Form<PREC>::S* __restrict__ b, const Geom& g, const ModelParams& p,
@@ -1787,8 +1784,7 @@ __device__ __forceinline__ void strip_wave(const typename Form<PREC>::S* __restr
 	// row x from rows x-1 (w0), x (w1, beside-the-strip h1) and x+1 (w2);
 	// row x+2 goes to w3 and h3
 	auto row = [&](int x, const S* w0, const S* w1, const S* w2, S* w3, const S h1, S& h3) {
-		// (the multi-phase march, with short chunks, skips the load it does not need)
-		if (KIND != 4 || x + 1 < xe) load_row(x + 2, w3, h3);
+		load_row(x + 2, w3, h3);
 		typename F::Sum sum = 0;
 		if (KIND == 1 || KIND == 3) {
 #pragma unroll
@@ -1801,71 +1797,28 @@ __device__ __forceinline__ void strip_wave(const typename Form<PREC>::S* __restr
 			if (out) gd = normal_deviate_cached(p.seed, p.step, x, (uint32_t)c, nkx, nkeep);
 			nkx = hit ? -1 : (x ^ 1);
 		}
-		if constexpr (KIND == 4) {
-			S phi[Q], lap[Q];
-			uint32_t act = 0;
-			S cnt = 0;
 #pragma unroll
-			for (int j = 0; j < Q; j++) {
-				const S y = w1[j];
-				const S yl = from_prev(y, lane_value(h1, j)), yh = from_next(y, lane_value(h1, Q + j));
-				phi[j] = y;
-				const bool on = y > S(0) || w2[j] > S(0) || w0[j] > S(0) || yh > S(0) || yl > S(0);
-				typename F::L l = F::lap_zero();
-				if (on) {
-					act |= 1u << j;
-					cnt += S(1);
-					F::lap_add(l, g.w[0], g.wf[0], w2[j], y, w0[j]);
-					F::lap_add(l, g.w[1], g.wf[1], yh, y, yl);
-				}
-				lap[j] = l;
-			}
-			if (cnt >= S(2)) gga_node<PREC, Q>(phi, lap, act, cnt, Q, p);
-			if (out) {
-#pragma unroll
-				for (int j = 0; j < Q; j++) (b + j * N)[o] = phi[j];
-			}
-		} else {
-#pragma unroll
-			for (int j = 0; j < Q; j++) {
-				const S y = w1[j];
-				const S yl = from_prev(y, lane_value(h1, j)), yh = from_next(y, lane_value(h1, Q + j));
-				typename F::L lap = F::lap_zero();
-				F::lap_add(lap, g.w[0], g.wf[0], w2[j], y, w0[j]);
-				F::lap_add(lap, g.w[1], g.wf[1], yh, y, yl);
-				if (out)
-					(b + j * N)[o] = KIND == 1 ? F::gg(y, sum, lap, p)
-					                 : KIND == 2 ? F::ac_noise(y, lap, gd, p)
-					                 : KIND == 3 ? (j == 0 ? y : F::gg(y, sum, lap, p))
-					                             : F::ac(y, lap, p);
-			}
+		for (int j = 0; j < Q; j++) {
+			const S y = w1[j];
+			const S yl = from_prev(y, lane_value(h1, j)), yh = from_next(y, lane_value(h1, Q + j));
+			typename F::L lap = F::lap_zero();
+			F::lap_add(lap, g.w[0], g.wf[0], w2[j], y, w0[j]);
+			F::lap_add(lap, g.w[1], g.wf[1], yh, y, yl);
+			if (out)
+				(b + j * N)[o] = KIND == 1 ? F::gg(y, sum, lap, p)
+				                 : KIND == 2 ? F::ac_noise(y, lap, gd, p)
+				                 : KIND == 3 ? (j == 0 ? y : F::gg(y, sum, lap, p))
+				                             : F::ac(y, lap, p);
 		}
 	};
-	if constexpr (KIND == 4) {
-		// the multi-phase body is large: four copies of it overflow the
-		// instruction cache, so one row per iteration and the slots advance
-		// by copies
-		for (int x = xb; x < xe; x++) {
-			row(x, wa, wb, wc, wd, hb, hd);
-#pragma unroll
-			for (int j = 0; j < Q; j++) {
-				wa[j] = wb[j];
-				wb[j] = wc[j];
-				wc[j] = wd[j];
-			}
-			hb = hc;
-			hc = hd;
-		}
-	} else {
-		for (int x = xb; x < xe; x += 4) {
-			row(x, wa, wb, wc, wd, hb, hd);
-			if (x + 1 >= xe) break;
-			row(x + 1, wb, wc, wd, wa, hc, ha);
-			if (x + 2 >= xe) break;
-			row(x + 2, wc, wd, wa, wb, hd, hb);
-			if (x + 3 >= xe) break;
-			row(x + 3, wd, wa, wb, wc, ha, hc);
-		}
+	for (int x = xb; x < xe; x += 4) {
+		row(x, wa, wb, wc, wd, hb, hd);
+		if (x + 1 >= xe) break;
+		row(x + 1, wb, wc, wd, wa, hc, ha);
+		if (x + 2 >= xe) break;
+		row(x + 2, wc, wd, wa, wb, hd, hb);
+		if (x + 3 >= xe) break;
+		row(x + 3, wd, wa, wb, wc, ha, hc);
 	}
 }
 
