@@ -23,8 +23,9 @@
 //     in launches of their own). 3-D members of 2^21 nodes or more fill the
 //     GPU on their own: they run the single-grid kernels instead (for
 //     periodic Cahn-Hilliard two steps per pass), one launch per member and
-//     pass, on a second compute stream, so they overlap the batch launches
-//     (both streams at the default priority). A round is planned on the host
+//     pass, on a second compute stream, so they overlap the batch launches,
+//     and half of those run on a third between a fork and a join (all streams
+//     at the default priority). A round is planned on the host
 //     and queued on the
 //     compute stream; up to two rounds are queued ahead, so the device does
 //     not wait for the host between rounds;
@@ -123,6 +124,8 @@ struct mmspx_server {
 	std::chrono::steady_clock::time_point t0;
 	hipStream_t st = nullptr;   // compute (worker): batch launches
 	hipStream_t st2 = nullptr;  // compute (worker): the large members' single-grid launches
+	hipStream_t st3 = nullptr;  // compute (worker): half of a round's batch launches, between fork and join
+	hipEvent_t fork = nullptr, join = nullptr;
 	hipStream_t ust = nullptr;  // uploads
 	hipStream_t dst = nullptr;  // downloads
 	hipMemPool_t pool = nullptr;
@@ -375,19 +378,35 @@ static int enqueue_round(mmspx_server* sv)
 	}
 	MMSPX_HIP(hipMemcpyAsync(sl.d_mem, sl.h_mem, sizeof(BMember) * act.size(), hipMemcpyHostToDevice, sv->st));
 	MMSPX_HIP(hipMemcpyAsync(sl.d_items, sl.h_items, sizeof(BItem) * (size_t)total, hipMemcpyHostToDevice, sv->st));
+	// The chains of launches (one per form and dimension) are independent, and a
+	// chain of small members leaves most of the GPU idle: the 3-D members of one
+	// form and the 2-D ones of the other run on a second stream, which starts
+	// behind the work lists' copies and which the compute stream waits for, so
+	// whatever is queued behind the round sees all of it done (16 requests of 21^3
+	// to 125^3 and 70^2 to 293^2 nodes: 15.7 ms on one stream, 12.6 on two)
+	const bool forked = (n2[0] > 0 || n3[1] > 0) && (n3[0] > 0 || n2[1] > 0);
+	if (forked) {
+		MMSPX_HIP(hipEventRecord(sv->fork, sv->st));
+		MMSPX_HIP(hipStreamWaitEvent(sv->st3, sv->fork, 0));
+	}
 	int64_t launches = 0;
 	int passes[2][2];  // by group and dimension
 	for (int grp = 0; grp < 2; grp++) {
 		for (int dim = 2; dim <= 3; dim++) {
+			const hipStream_t st = forked && (grp == 1) == (dim == 3) ? sv->st3 : sv->st;
 			const int n = dim == 2 ? n2[grp] : n3[grp], spp = batch_steps_per_pass(sv->cfg.model, tile[grp], dim);
 			const BItem* it = sl.d_items + off[grp] + (dim == 2 ? 0 : n2[grp]);
 			passes[grp][dim - 2] = (steps + spp - 1) / spp;
 			for (int k = 0; n > 0 && k * spp < steps; k++) {
-				rc = launch_batch_pass(sv->cfg.model, form[grp], 1, tile[grp], sl.d_mem, it, n, dim, k & 1, sv->cus, sv->st,
+				rc = launch_batch_pass(sv->cfg.model, form[grp], 1, tile[grp], sl.d_mem, it, n, dim, k & 1, sv->cus, st,
 				                       &launches, std::min(spp, steps - k * spp));
 				if (rc) return rc;
 			}
 		}
+	}
+	if (forked) {
+		MMSPX_HIP(hipEventRecord(sv->join, sv->st3));
+		MMSPX_HIP(hipStreamWaitEvent(sv->st, sv->join, 0));
 	}
 	for (Request* r : act)
 		if (!r->solo) r->cur ^= passes[r->prec != sv->cfg.precision][r->g.dim == 3 ? 1 : 0] & 1;
@@ -579,6 +598,7 @@ static void worker_main(mmspx_server* sv)
 		if (rc == 0) continue;
 		(void)hipStreamSynchronize(sv->st);
 		(void)hipStreamSynchronize(sv->st2);
+		(void)hipStreamSynchronize(sv->st3);
 		if (rc == 1) break;
 		// a device error: fail every request not yet finished and stop serving
 		std::lock_guard<std::mutex> lk(sv->mu);
@@ -613,6 +633,9 @@ int mmspx_server_create(const mmspx_server_config* cfg, mmspx_server** out)
 	int rc = 0;
 	if (hipGetDevice(&sv->device) != hipSuccess || hipStreamCreateWithFlags(&sv->st, hipStreamNonBlocking) != hipSuccess ||
 	    hipStreamCreateWithFlags(&sv->st2, hipStreamNonBlocking) != hipSuccess ||
+	    hipStreamCreateWithFlags(&sv->st3, hipStreamNonBlocking) != hipSuccess ||
+	    hipEventCreateWithFlags(&sv->fork, hipEventDisableTiming) != hipSuccess ||
+	    hipEventCreateWithFlags(&sv->join, hipEventDisableTiming) != hipSuccess ||
 	    hipStreamCreateWithFlags(&sv->ust, hipStreamNonBlocking) != hipSuccess ||
 	    hipStreamCreateWithFlags(&sv->dst, hipStreamNonBlocking) != hipSuccess)
 		rc = fail(MMSPX_EDEVICE, "HIP stream setup failed");
@@ -642,6 +665,9 @@ int mmspx_server_create(const mmspx_server_config* cfg, mmspx_server** out)
 		if (sv->pool) (void)hipMemPoolDestroy(sv->pool);
 		if (sv->st) (void)hipStreamDestroy(sv->st);
 		if (sv->st2) (void)hipStreamDestroy(sv->st2);
+		if (sv->st3) (void)hipStreamDestroy(sv->st3);
+		if (sv->fork) (void)hipEventDestroy(sv->fork);
+		if (sv->join) (void)hipEventDestroy(sv->join);
 		if (sv->ust) (void)hipStreamDestroy(sv->ust);
 		if (sv->dst) (void)hipStreamDestroy(sv->dst);
 		delete sv;
@@ -670,6 +696,7 @@ void mmspx_server_destroy(mmspx_server* sv)
 	if (sv->downloader.joinable()) sv->downloader.join();
 	(void)hipStreamSynchronize(sv->st);
 	(void)hipStreamSynchronize(sv->st2);
+	(void)hipStreamSynchronize(sv->st3);
 	(void)hipStreamSynchronize(sv->ust);
 	(void)hipStreamSynchronize(sv->dst);
 	std::set<Request*> fetched;  // fetched, still listed by rounds never retired
@@ -699,6 +726,9 @@ void mmspx_server_destroy(mmspx_server* sv)
 	(void)hipMemPoolDestroy(sv->pool);
 	(void)hipStreamDestroy(sv->st);
 	(void)hipStreamDestroy(sv->st2);
+	(void)hipStreamDestroy(sv->st3);
+	(void)hipEventDestroy(sv->fork);
+	(void)hipEventDestroy(sv->join);
 	(void)hipStreamDestroy(sv->ust);
 	(void)hipStreamDestroy(sv->dst);
 	delete sv;
