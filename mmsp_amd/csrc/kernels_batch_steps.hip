@@ -39,7 +39,7 @@ __global__ void __launch_bounds__(256) steps2d_batch(const BMember* __restrict__
 	const BItem w = items[it];
 	const BMember m = mem[w.m];
 	const int src = (parity + m.phase) & 1;
-	steps2d<PREC, MODEL, L, EDGES, false, FULL>(member_buf<S>(m, src), member_buf<S>(m, src ^ 1), m.g, m.p, w.z0, w.xb, w.xe,
+	steps2d<PREC, MODEL, L, EDGES, 0, FULL>(member_buf<S>(m, src), member_buf<S>(m, src ^ 1), m.g, m.p, w.z0, w.xb, w.xe,
 	                                            levels);
 }
 
@@ -53,7 +53,7 @@ __global__ void __launch_bounds__(NT) march4_batch(const BMember* __restrict__ m
 	const BItem w = items[it];
 	const BMember m = mem[w.m];
 	const int src = (parity + m.phase) & 1;
-	march4<PREC, MODEL, TY, TZ, NT, LEVELS, false>(member_buf<S>(m, src), member_buf<S>(m, src ^ 1), m.g, m.p, w.y0, w.z0, w.xb,
+	march4<PREC, MODEL, TY, TZ, NT, LEVELS, 0>(member_buf<S>(m, src), member_buf<S>(m, src ^ 1), m.g, m.p, w.y0, w.z0, w.xb,
 	                                               w.xe);
 }
 

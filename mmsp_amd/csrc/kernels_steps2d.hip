@@ -12,7 +12,7 @@ namespace mmspx {
 // strip-fastest and an XCD takes a contiguous run of them, so neighbouring
 // strips of the same rows share their halo columns in one L2. The item is
 // made wave-uniform so that the march's row bookkeeping runs on the scalar unit.
-template <int PREC, int MODEL, int L, bool EDGES, bool UNIT, bool FULL>
+template <int PREC, int MODEL, int L, bool EDGES, int UNIT, bool FULL>
 __global__ void __launch_bounds__(256) steps2d_k(const typename Form<PREC>::S* __restrict__ a,
                                                  typename Form<PREC>::S* __restrict__ b, Geom g, ModelParams p,
                                                  int chunk_len, int strips, int nitems, int levels)
@@ -26,7 +26,7 @@ __global__ void __launch_bounds__(256) steps2d_k(const typename Form<PREC>::S* _
 	steps2d<PREC, MODEL, L, EDGES, UNIT, FULL>(a, b, g, p, s * (64 - 2 * L), xb, min(xb + chunk_len, g.n[0]), levels);
 }
 
-template <int PREC, int MODEL, int L, bool EDGES, bool UNIT, bool FULL>
+template <int PREC, int MODEL, int L, bool EDGES, int UNIT, bool FULL>
 static int launch_body(const Geom& g, const ModelParams& p, const void* a, void* b, hipStream_t st, int chunk,
                        int levels)
 {
@@ -40,7 +40,7 @@ static int launch_body(const Geom& g, const ModelParams& p, const void* a, void*
 	return 0;
 }
 
-template <int PREC, int MODEL, bool EDGES, bool UNIT>
+template <int PREC, int MODEL, bool EDGES, int UNIT>
 static int launch_unit(const Geom& g, const ModelParams& p, const void* a, void* b, hipStream_t st, int chunk,
                        int levels)
 {
@@ -48,21 +48,24 @@ static int launch_unit(const Geom& g, const ModelParams& p, const void* a, void*
 	// steps branches over the levels past its last one
 	if (levels == 8) return launch_body<PREC, MODEL, 8, EDGES, UNIT, true>(g, p, a, b, st, chunk, levels);
 	if (levels == 4) return launch_body<PREC, MODEL, 4, EDGES, UNIT, true>(g, p, a, b, st, chunk, levels);
-	return launch_body<PREC, MODEL, 8, EDGES, false, false>(g, p, a, b, st, chunk, levels);
+	return launch_body<PREC, MODEL, 8, EDGES, 0, false>(g, p, a, b, st, chunk, levels);
 }
 
 template <int PREC, int MODEL>
 static int launch_model(const Geom& g, const ModelParams& p, const void* a, void* b, hipStream_t st, int chunk,
                         int levels)
 {
-	const bool unit = g.w[0] == 1.0 && g.w[1] == 1.0 && g.wf[0] == 1.0f && g.wf[1] == 1.0f;
+	int unit = g.w[0] == 1.0 && g.w[1] == 1.0 && g.wf[0] == 1.0f && g.wf[1] == 1.0f;
+	if (unit && (MODEL == S2_CH_DW ? p.kappa == 1.0 && p.kappaf == 1.0f : unit_coefficients(p))) unit = 2;
 	bool edges = false;
 	for (int k = 0; k < 2; k++) edges |= g.b0[k] != MMSPX_PERIODIC || g.b1[k] != MMSPX_PERIODIC;
 	if (edges)
-		return unit ? launch_unit<PREC, MODEL, true, true>(g, p, a, b, st, chunk, levels)
-		            : launch_unit<PREC, MODEL, true, false>(g, p, a, b, st, chunk, levels);
-	return unit ? launch_unit<PREC, MODEL, false, true>(g, p, a, b, st, chunk, levels)
-	            : launch_unit<PREC, MODEL, false, false>(g, p, a, b, st, chunk, levels);
+		return unit == 2 ? launch_unit<PREC, MODEL, true, 2>(g, p, a, b, st, chunk, levels)
+		       : unit    ? launch_unit<PREC, MODEL, true, 1>(g, p, a, b, st, chunk, levels)
+		                 : launch_unit<PREC, MODEL, true, 0>(g, p, a, b, st, chunk, levels);
+	return unit == 2 ? launch_unit<PREC, MODEL, false, 2>(g, p, a, b, st, chunk, levels)
+	       : unit    ? launch_unit<PREC, MODEL, false, 1>(g, p, a, b, st, chunk, levels)
+	                 : launch_unit<PREC, MODEL, false, 0>(g, p, a, b, st, chunk, levels);
 }
 
 template <int PREC>

@@ -72,10 +72,11 @@ constexpr int lds_pitch(int cols, int bz, int elem)
 	return best;
 }
 
-// LEVELS < 4: a last pass of fewer steps, level LEVELS is written. UNIT: every
-// grid weight is 1 and, for Cahn-Hilliard, so is the gradient coefficient (the
-// multiplications by them are left out; the bits are the same).
-template <int PREC, int MODEL, int TY, int TZ, int NT, int LEVELS, bool UNIT>
+// LEVELS < 4: a last pass of fewer steps, level LEVELS is written. UNIT 1: every
+// grid weight is 1 and, for Cahn-Hilliard, so is the gradient coefficient, 2: so
+// is every coefficient (the multiplications by them are left out; the bits are
+// the same).
+template <int PREC, int MODEL, int TY, int TZ, int NT, int LEVELS, int UNIT>
 __device__ __forceinline__ void march4(const typename Form<PREC>::S* __restrict__ a,
                                        typename Form<PREC>::S* __restrict__ b, const Geom& g, const ModelParams& p,
                                        int y0, int z0, int xb, int xe)
@@ -182,23 +183,24 @@ __device__ __forceinline__ void march4(const typename Form<PREC>::S* __restrict_
 		const int A = odd ? W / 2 : 0, B = odd ? 1 : W / 2, Lc = odd ? 0 : W / 2 - 1, Rc = odd ? W / 2 + 1 : 1;
 		const S u0 = q[A - W], u1 = q[B - W], d0 = q[A + 2 * W], d1 = q[B + 2 * W];
 		const S l0 = q[Lc], l1 = q[Lc + W], h0 = q[Rc], h1 = q[Rc + W];
-		o[0] = lap3<PREC, UNIT, MODEL == S2_CH>(g, h[0], l[0], m[2], u0, m[1], l0, m[0]);
-		o[1] = lap3<PREC, UNIT, MODEL == S2_CH>(g, h[1], l[1], m[3], u1, h0, m[0], m[1]);
-		o[2] = lap3<PREC, UNIT, MODEL == S2_CH>(g, h[2], l[2], d0, m[0], m[3], l1, m[2]);
-		o[3] = lap3<PREC, UNIT, MODEL == S2_CH>(g, h[3], l[3], d1, m[1], h1, m[2], m[3]);
+		o[0] = lap3<PREC, UNIT != 0, MODEL == S2_CH>(g, h[0], l[0], m[2], u0, m[1], l0, m[0]);
+		o[1] = lap3<PREC, UNIT != 0, MODEL == S2_CH>(g, h[1], l[1], m[3], u1, h0, m[0], m[1]);
+		o[2] = lap3<PREC, UNIT != 0, MODEL == S2_CH>(g, h[2], l[2], d0, m[0], m[3], l1, m[2]);
+		o[3] = lap3<PREC, UNIT != 0, MODEL == S2_CH>(g, h[3], l[3], d1, m[1], h1, m[2], m[3]);
 	};
 	auto mu = [&](S c, typename F::L lap) -> S {
 		if constexpr (MODEL == S2_CH_DW && UNIT) return F::mu_dw1(c, lap);
 		else if constexpr (MODEL == S2_CH_DW) return F::mu_dw(c, lap, p);
-		else if constexpr (UNIT) return F::mu_poly1(c, lap, p);
+		else if constexpr (UNIT == 2) return mu_unit<PREC>(c, lap);
+		else if constexpr (UNIT == 1) return F::mu_poly1(c, lap, p);
 		else return F::mu_poly(c, lap, p);
 	};
 	auto odd = [&](S y, typename F::L lap) -> S {
-		if constexpr (MODEL == S2_AC) return F::ac(y, lap, p);
+		if constexpr (MODEL == S2_AC) return UNIT == 2 ? ac_unit<PREC>(y, lap, p) : F::ac(y, lap, p);
 		else return mu(y, lap);
 	};
 	auto even = [&](S y, typename F::L lap, S c) -> S {
-		if constexpr (MODEL == S2_AC) return F::ac(y, lap, p);
+		if constexpr (MODEL == S2_AC) return UNIT == 2 ? ac_unit<PREC>(y, lap, p) : F::ac(y, lap, p);
 		else return F::ch(c, lap, p);
 	};
 

@@ -9,7 +9,7 @@
 namespace mmspx {
 
 // One workgroup per (tile, chunk), XCD-contiguous runs as the other marches.
-template <int PREC, int MODEL, int TY, int TZ, int NT, int LEVELS, bool UNIT>
+template <int PREC, int MODEL, int TY, int TZ, int NT, int LEVELS, int UNIT>
 __global__ void __launch_bounds__(NT) march4_k(const typename Form<PREC>::S* __restrict__ a,
                                                typename Form<PREC>::S* __restrict__ b, Geom g, ModelParams p,
                                                int chunk_len, int tiles_y, int tiles_z, int ntiles)
@@ -24,7 +24,7 @@ __global__ void __launch_bounds__(NT) march4_k(const typename Form<PREC>::S* __r
 	march4<PREC, MODEL, TY, TZ, NT, LEVELS, UNIT>(a, b, g, p, ty * TY, tz * TZ, xb, min(xb + chunk_len, g.n[0]));
 }
 
-template <int PREC, int MODEL, int TY, int TZ, int NT, int LEVELS, bool UNIT>
+template <int PREC, int MODEL, int TY, int TZ, int NT, int LEVELS, int UNIT>
 static int launch_march4_body(const Geom& g, const ModelParams& p, const void* a, void* b, hipStream_t st, int chunk)
 {
 	using S = typename Form<PREC>::S;
@@ -37,7 +37,7 @@ static int launch_march4_body(const Geom& g, const ModelParams& p, const void* a
 	return 0;
 }
 
-template <int PREC, int MODEL, int NW, int R, int LEVELS, bool UNIT>
+template <int PREC, int MODEL, int NW, int R, int LEVELS, int UNIT>
 __global__ void __launch_bounds__(64 * NW) wmarch4_k(const typename Form<PREC>::S* __restrict__ a,
                                                      typename Form<PREC>::S* __restrict__ b, Geom g, ModelParams p,
                                                      int chunk_len, int tiles_y, int tiles_z, int ntiles)
@@ -52,7 +52,7 @@ __global__ void __launch_bounds__(64 * NW) wmarch4_k(const typename Form<PREC>::
 	wmarch4<PREC, MODEL, NW, R, LEVELS, UNIT>(a, b, g, p, ty * (NW * R - 6), tz * 56, xb, min(xb + chunk_len, g.n[0]));
 }
 
-template <int PREC, int MODEL, int NW, int R, int LEVELS, bool UNIT>
+template <int PREC, int MODEL, int NW, int R, int LEVELS, int UNIT>
 static int launch_wmarch4_body(const Geom& g, const ModelParams& p, const void* a, void* b, hipStream_t st, int chunk)
 {
 	using S = typename Form<PREC>::S;
@@ -61,13 +61,13 @@ static int launch_wmarch4_body(const Geom& g, const ModelParams& p, const void* 
 	const int tiles_z = (g.n[2] + TZ - 1) / TZ;
 	const int ntiles = tiles_y * tiles_z * ((g.n[0] + chunk - 1) / chunk);
 	// a last pass of fewer steps multiplies by unit weights too
-	hipLaunchKernelGGL((wmarch4_k<PREC, MODEL, NW, R, LEVELS, UNIT && LEVELS == 4>), dim3((ntiles + 7) / 8 * 8),
+	hipLaunchKernelGGL((wmarch4_k<PREC, MODEL, NW, R, LEVELS, LEVELS == 4 ? UNIT : 0>), dim3((ntiles + 7) / 8 * 8),
 	                   dim3(64 * NW), 0, st, (const S*)a, (S*)b, g, p, chunk, tiles_y, tiles_z, ntiles);
 	MMSPX_HIP(hipGetLastError());
 	return 0;
 }
 
-template <int PREC, int MODEL, int LEVELS, bool UNIT>
+template <int PREC, int MODEL, int LEVELS, int UNIT>
 static int launch_march4_tile(const Geom& g, const ModelParams& p, const void* a, void* b, hipStream_t st,
                               const TuneChoice& t)
 {
@@ -95,16 +95,21 @@ template <int PREC, int MODEL>
 static int launch_march4_model(const Geom& g, const ModelParams& p, const void* a, void* b, hipStream_t st,
                                const TuneChoice& t, int nsteps)
 {
-	bool unit = true;
-	for (int k = 0; k < 3; k++) unit = unit && g.w[k] == 1.0 && g.wf[k] == 1.0f;
-	if (MODEL == S2_CH) unit = unit && p.K == 1.0 && p.Kf == 1.0f;
-	if (MODEL == S2_CH_DW) unit = unit && p.kappa == 1.0 && p.kappaf == 1.0f;
+	bool weights = true;
+	for (int k = 0; k < 3; k++) weights = weights && g.w[k] == 1.0 && g.wf[k] == 1.0f;
+	int unit = weights;
+	if (MODEL == S2_CH) unit = weights && p.K == 1.0 && p.Kf == 1.0f;
+	if (MODEL == S2_CH_DW) unit = weights && p.kappa == 1.0 && p.kappaf == 1.0f;
+	if (MODEL != S2_CH_DW && unit && unit_coefficients(p)) unit = 2;
 	const int levels = nsteps * (MODEL == S2_AC ? 1 : 2);
 	// fewer than four levels: a last pass of fewer steps
 	auto run = [&](auto lv) {
 		constexpr int L = decltype(lv)::value;
-		return unit ? launch_march4_tile<PREC, MODEL, L, true>(g, p, a, b, st, t)
-		            : launch_march4_tile<PREC, MODEL, L, false>(g, p, a, b, st, t);
+		if constexpr (MODEL != S2_CH_DW) {
+			if (unit == 2) return launch_march4_tile<PREC, MODEL, L, 2>(g, p, a, b, st, t);
+		}
+		return unit ? launch_march4_tile<PREC, MODEL, L, 1>(g, p, a, b, st, t)
+		            : launch_march4_tile<PREC, MODEL, L, 0>(g, p, a, b, st, t);
 	};
 	if (levels == 4) return run(std::integral_constant<int, 4>{});
 	if (levels == 2) return run(std::integral_constant<int, 2>{});

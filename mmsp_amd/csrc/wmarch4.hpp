@@ -51,7 +51,7 @@ __device__ __forceinline__ typename Form<PREC>::L wlap3(const Geom& g, typename 
 	return ((ZERO ? S(0) + tx : tx) + ty) + tz;
 }
 
-template <int PREC, int MODEL, int NW, int R, int LEVELS, bool UNIT>
+template <int PREC, int MODEL, int NW, int R, int LEVELS, int UNIT>
 __device__ __forceinline__ void wmarch4(const typename Form<PREC>::S* __restrict__ a,
                                         typename Form<PREC>::S* __restrict__ b, const Geom& g, const ModelParams& p,
                                         int y0, int z0, int xb, int xe)
@@ -121,21 +121,22 @@ __device__ __forceinline__ void wmarch4(const typename Form<PREC>::S* __restrict
 #pragma unroll
 		for (int k = 0; k < R; k++) {
 			const S yl = k > 0 ? m[k > 0 ? k - 1 : 0] : up[level], yh = k < R - 1 ? m[k < R - 1 ? k + 1 : 0] : dn[level];
-			value(k, wlap3<PREC, UNIT, MODEL == S2_CH>(g, h[k], l[k], yh, yl, m[k]));
+			value(k, wlap3<PREC, UNIT != 0, MODEL == S2_CH>(g, h[k], l[k], yh, yl, m[k]));
 		}
 	};
 	auto mu = [&](S c, typename F::L lap) -> S {
 		if constexpr (MODEL == S2_CH_DW && UNIT) return F::mu_dw1(c, lap);
 		else if constexpr (MODEL == S2_CH_DW) return F::mu_dw(c, lap, p);
-		else if constexpr (UNIT) return F::mu_poly1(c, lap, p);
+		else if constexpr (UNIT == 2) return mu_unit<PREC>(c, lap);
+		else if constexpr (UNIT == 1) return F::mu_poly1(c, lap, p);
 		else return F::mu_poly(c, lap, p);
 	};
 	auto odd = [&](S y, typename F::L lap) -> S {
-		if constexpr (MODEL == S2_AC) return F::ac(y, lap, p);
+		if constexpr (MODEL == S2_AC) return UNIT == 2 ? ac_unit<PREC>(y, lap, p) : F::ac(y, lap, p);
 		else return mu(y, lap);
 	};
 	auto even = [&](S y, typename F::L lap, S c) -> S {
-		if constexpr (MODEL == S2_AC) return F::ac(y, lap, p);
+		if constexpr (MODEL == S2_AC) return UNIT == 2 ? ac_unit<PREC>(y, lap, p) : F::ac(y, lap, p);
 		else return F::ch(c, lap, p);
 	};
 
