@@ -745,6 +745,10 @@ def main():
             "gg_aniso": "gga"}[w["model"]]
     if tile["variant"] != 2:
         kname = base + "_generic"
+    elif len(shape) == 3 and base == "gg" and tile["tz"] in (56, 58, 60):
+        kname = "fmarch"
+    elif len(shape) == 3 and tile["tz"] == 56:
+        kname = "wmarch4"
     elif len(shape) == 3 and tile["opt"] == 8:
         kname = "march3d"
     elif len(shape) == 3 and tile["opt"] == 12:
@@ -753,6 +757,10 @@ def main():
         kname = "ch_fused"
     elif base == "ow":
         kname = "ow_waves"
+    elif tile["opt"] in (13, 14):
+        kname = "steps2d"
+    elif tile["opt"] == 16:
+        kname = "fields2d"
     elif tile["opt"] == 2:
         kname = "wave_strips"
     elif tile["opt"] in (4, 5):
