@@ -37,8 +37,9 @@ static int launch_fmarch_body(const Geom& g, const ModelParams& p, const void* a
 	return 0;
 }
 
-// whole passes, and a last one of fewer steps (which multiplies by unit weights too)
-template <int PREC, int Q, int R, int L, int KIND>
+// whole passes, and a last one of fewer steps (which multiplies by unit weights
+// too); OWN: the number of those that has a tile of its own
+template <int PREC, int Q, int R, int L, int KIND, int OWN = 0>
 static int launch_fmarch_steps(const Geom& g, const ModelParams& p, const void* a, void* b, hipStream_t st, int chunk,
                                int nsteps)
 {
@@ -49,10 +50,10 @@ static int launch_fmarch_steps(const Geom& g, const ModelParams& p, const void* 
 		            : launch_fmarch_body<PREC, Q, KIND, R, L, L, false>(g, p, a, b, st, chunk);
 	}
 	if (nsteps == 1) return launch_fmarch_body<PREC, Q, KIND, R, L, 1, false>(g, p, a, b, st, chunk);
-	if constexpr (L > 2) {
+	if constexpr (L > 2 && OWN != 2) {
 		if (nsteps == 2) return launch_fmarch_body<PREC, Q, KIND, R, L, 2, false>(g, p, a, b, st, chunk);
 	}
-	if constexpr (L > 3) {
+	if constexpr (L > 3 && OWN != 3) {
 		if (nsteps == 3) return launch_fmarch_body<PREC, Q, KIND, R, L, 3, false>(g, p, a, b, st, chunk);
 	}
 	return fail(MMSPX_EINVAL, "more steps than a pass of the field march takes");
@@ -67,17 +68,17 @@ static int launch_fmarch_prec(const Geom& g, const ModelParams& p, const void* a
 		return g.fields == q && t.ty == 16 / q * r - 2 * (l - 1) && t.tz == 64 - 2 * l;
 	};
 	if constexpr (PREC == MMSPX_F32) {
-		if (is(8, 8, 3)) return launch_fmarch_steps<PREC, 8, 8, 3, KIND>(g, p, a, b, st, t.chunk, nsteps);
+		if (is(8, 8, 3)) return launch_fmarch_steps<PREC, 8, 8, 3, KIND, 2>(g, p, a, b, st, t.chunk, nsteps);
 		if (is(8, 12, 2)) return launch_fmarch_steps<PREC, 8, 12, 2, KIND>(g, p, a, b, st, t.chunk, nsteps);
-		if (is(4, 6, 4)) return launch_fmarch_steps<PREC, 4, 6, 4, KIND>(g, p, a, b, st, t.chunk, nsteps);
+		if (is(4, 6, 4)) return launch_fmarch_steps<PREC, 4, 6, 4, KIND, 3>(g, p, a, b, st, t.chunk, nsteps);
 		if (is(4, 8, 3)) return launch_fmarch_steps<PREC, 4, 8, 3, KIND>(g, p, a, b, st, t.chunk, nsteps);
 		if (is(2, 4, 4)) return launch_fmarch_steps<PREC, 2, 4, 4, KIND>(g, p, a, b, st, t.chunk, nsteps);
 	} else {
 		if (is(8, 5, 2)) return launch_fmarch_steps<PREC, 8, 5, 2, KIND>(g, p, a, b, st, t.chunk, nsteps);
 		if (is(8, 6, 2)) return launch_fmarch_steps<PREC, 8, 6, 2, KIND>(g, p, a, b, st, t.chunk, nsteps);
 		if (is(4, 6, 2)) return launch_fmarch_steps<PREC, 4, 6, 2, KIND>(g, p, a, b, st, t.chunk, nsteps);
-		if (is(4, 4, 3)) return launch_fmarch_steps<PREC, 4, 4, 3, KIND>(g, p, a, b, st, t.chunk, nsteps);
-		if (is(2, 3, 4)) return launch_fmarch_steps<PREC, 2, 3, 4, KIND>(g, p, a, b, st, t.chunk, nsteps);
+		if (is(4, 4, 3)) return launch_fmarch_steps<PREC, 4, 4, 3, KIND, 2>(g, p, a, b, st, t.chunk, nsteps);
+		if (is(2, 3, 4)) return launch_fmarch_steps<PREC, 2, 3, 4, KIND, 3>(g, p, a, b, st, t.chunk, nsteps);
 		if (is(2, 4, 3)) return launch_fmarch_steps<PREC, 2, 4, 3, KIND>(g, p, a, b, st, t.chunk, nsteps);
 	}
 	return fail(MMSPX_EINVAL, "no field march compiled for this tile and field count");

@@ -68,6 +68,33 @@ static double plane_march_us(const Geom& g, int prec, int body)
 	return 0.0;
 }
 
+// us of a pass on tile t with its best chunk
+static double best_pass(const Geom& g, const FieldTile& t, TuneChoice* out)
+{
+	const int L = (64 - t.tz) / 2;
+	const double node_bytes = (double)t.fields * (t.prec == MMSPX_F64 ? 8 : 4);
+	const double plane_bytes = ((t.ty + 2 * L) * 64.0 + (double)t.ty * t.tz) * node_bytes;
+	const int64_t tiles = (int64_t)((g.n[1] + t.ty - 1) / t.ty) * ((g.n[2] + t.tz - 1) / t.tz);
+	double best = 1e300;
+	auto take = [&](int c) {
+		const int64_t wgs = tiles * ((g.n[0] + c - 1) / c);
+		const int planes = c + 2 * (L - 1);
+		const double work = t.plane * planes * (double)((wgs + 255) / 256);
+		const double move = plane_bytes * planes * (double)wgs / (t.tbs * 1e6);
+		const double us = t.t0 + std::max(work, move);
+		if (us < best) {
+			best = us;
+			*out = TuneChoice{2, t.ty, t.tz, c, 17};
+		}
+	};
+	for (int c = 3; c <= 16; c++) take(c);
+	for (int n = 1; n <= 32; n++) {
+		const int c = (g.n[0] + n - 1) / n;
+		if (c > 16 && c <= 512) take(c);
+	}
+	return best;
+}
+
 // Tile and chunk by the cost above, where that is 7 % less than the plane
 // marches take (both fitted to a sweep of 12 grids from 40 x 24 x 128 to 256^3,
 // within 10 %). us per step, plane march and this: 256^3 x 8 FP32 212 and 167,
@@ -82,25 +109,11 @@ bool fmarch_choice(const Geom& g, int prec, int model, TuneChoice* out)
 	double best = 1e300;
 	for (const FieldTile& t : kFieldTiles) {
 		if (t.prec != prec || t.fields != g.fields) continue;
-		const int L = (64 - t.tz) / 2;
-		const double node_bytes = (double)t.fields * (prec == MMSPX_F64 ? 8 : 4);
-		const double plane_bytes = ((t.ty + 2 * L) * 64.0 + (double)t.ty * t.tz) * node_bytes;
-		const int64_t tiles = (int64_t)((g.n[1] + t.ty - 1) / t.ty) * ((g.n[2] + t.tz - 1) / t.tz);
-		auto take = [&](int c) {
-			const int64_t wgs = tiles * ((g.n[0] + c - 1) / c);
-			const int planes = c + 2 * (L - 1);
-			const double work = t.plane * planes * (double)((wgs + 255) / 256);
-			const double move = plane_bytes * planes * (double)wgs / (t.tbs * 1e6);
-			const double us = (t.t0 + std::max(work, move)) / L;
-			if (us < best) {
-				best = us;
-				*out = TuneChoice{2, t.ty, t.tz, c, 17};
-			}
-		};
-		for (int c = 3; c <= 16; c++) take(c);
-		for (int n = 1; n <= 32; n++) {
-			const int c = (g.n[0] + n - 1) / n;
-			if (c > 16 && c <= 512) take(c);
+		TuneChoice c;
+		const double us = best_pass(g, t, &c) / fmarch_steps(c);
+		if (us < best) {
+			best = us;
+			*out = c;
 		}
 	}
 	return best < 0.93 * plane_march_us(g, prec, one_step_choice(g, prec, model).opt == 12 ? 12 : 8);
@@ -118,12 +131,21 @@ int fmarch_candidates(const Geom& g, int prec, int model, TuneChoice* out, int m
 }
 
 int launch_fmarch(const Geom& g, int prec, const ModelParams& p, const void* a, void* b, hipStream_t st,
-                  const TuneChoice& t, int nsteps)
+                  const TuneChoice& tile, int nsteps)
 {
 	if (!fmarch_supported(g, prec, p.model))
 		return fail(MMSPX_EUNSUPPORTED, "the field march takes periodic 3-D grain growth and Zener pinning with 2, 4 or 8 "
 		                                "fields in the MMSPX_F64 and MMSPX_F32 forms");
-	if (t.chunk < 1 || nsteps < 1) return fail(MMSPX_EINVAL, "bad chunk or step count");
+	if (tile.chunk < 1 || nsteps < 1) return fail(MMSPX_EINVAL, "bad chunk or step count");
+	// a last pass of fewer steps: the tile made for that many, if there is one
+	// (two steps of 256^3 x 8 FP32: 457 us on the three-step tile, 369 on its own)
+	TuneChoice t = tile;
+	if (nsteps < fmarch_steps(tile))
+		for (const FieldTile& o : kFieldTiles)
+			if (o.prec == prec && o.fields == g.fields && (64 - o.tz) / 2 == nsteps) {
+				best_pass(g, o, &t);
+				break;
+			}
 	if (prec == MMSPX_F64)
 		return p.model == MMSPX_ZENER ? launch_fmarch_f64_zener(g, p, a, b, st, t, nsteps)
 		                              : launch_fmarch_f64_gg(g, p, a, b, st, t, nsteps);
