@@ -546,9 +546,13 @@ __device__ __forceinline__ void gga_project(typename Form<PREC>::S (&phi)[QMAX],
 // a node with at most 4 fields present packs them, in ascending order, into 4
 // slots first: the same additions in the same order as the full loops (which
 // skip the absent fields), on a quarter of the field triples.
-template <int PREC, int QMAX>
+// ST > 0: the packing goes through 8 LDS slots of the thread's own, ST apart,
+// instead of selects over every pair of field and slot (plane march of 128^3 x 8
+// fields: FP64 108.5 -> 101.4 us per step, FP32 73.6 -> 70.9).
+template <int PREC, int QMAX, int ST = 0>
 __device__ __forceinline__ void gga_node(typename Form<PREC>::S (&phi)[QMAX], const typename Form<PREC>::S (&lap)[QMAX],
-                                         uint32_t act, typename Form<PREC>::S cnt, int Q, const ModelParams& p)
+                                         uint32_t act, typename Form<PREC>::S cnt, int Q, const ModelParams& p,
+                                         typename Form<PREC>::S* slots = nullptr)
 {
 	using S = typename Form<PREC>::S;
 	constexpr int K = 4;
@@ -556,6 +560,35 @@ __device__ __forceinline__ void gga_node(typename Form<PREC>::S (&phi)[QMAX], co
 	if constexpr (QMAX > K && QMAX <= 8) {
 		if (cnt <= S(K)) {
 			S cphi[K], clap[K], cdp[K];
+			if constexpr (ST > 0) {
+				S* at = slots;
+#pragma unroll
+				for (int f = 0; f < QMAX; f++)
+					if (act >> f & 1u) {
+						at[0] = phi[f];
+						at[K * ST] = lap[f];
+						at += ST;
+					}
+#pragma unroll
+				for (int s = 0; s < K; s++) {
+					cphi[s] = slots[s * ST];
+					clap[s] = slots[(K + s) * ST];
+				}
+				gga_rates4<PREC>(cphi, clap, (int)cnt, p, cdp);
+#pragma unroll
+				for (int s = 0; s < K; s++) slots[s * ST] = cdp[s];
+				at = slots;
+#pragma unroll
+				for (int f = 0; f < QMAX; f++) {
+					dp[f] = 0;
+					if (act >> f & 1u) {
+						dp[f] = at[0];
+						at += ST;
+					}
+				}
+				gga_project<PREC, QMAX>(phi, dp, cnt, Q, p);
+				return;
+			}
 #pragma unroll
 			for (int s = 0; s < K; s++) cphi[s] = clap[s] = 0;
 #pragma unroll

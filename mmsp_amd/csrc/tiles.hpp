@@ -640,6 +640,7 @@ __device__ __forceinline__ void march3d(const typename Form<PREC>::S* __restrict
 	constexpr int PN = PY * PZ, ON = TY * TZ, RN = PN - ON;
 	constexpr int M = (ON + NT - 1) / NT;
 	constexpr int MR = (RN + NT - 1) / NT;
+	__shared__ S slots[KIND == 4 && Q > 4 ? 8 * NT : 1];  // multi-phase: packed fields of a node
 	__shared__ S lt[2][Q][PN];
 
 	const int nx = g.n[0], ny = g.n[1], nz = g.n[2];
@@ -795,7 +796,11 @@ __device__ __forceinline__ void march3d(const typename Form<PREC>::S* __restrict
 					}
 					lap[q] = l;
 				}
-				if (cnt >= S(2)) gga_node<PREC, Q>(phi, lap, act, cnt, Q, p);
+				if constexpr (Q > 4) {
+					if (cnt >= S(2)) gga_node<PREC, Q, NT>(phi, lap, act, cnt, Q, p, slots + threadIdx.x);
+				} else {
+					if (cnt >= S(2)) gga_node<PREC, Q>(phi, lap, act, cnt, Q, p);
+				}
 #pragma unroll
 				for (int q = 0; q < Q; q++) dst[q * N + ooff[k]] = phi[q];
 				continue;
