@@ -23,12 +23,11 @@
 //     in launches of their own). 3-D members of 2^21 nodes or more fill the
 //     GPU on their own: they run the single-grid kernels instead (for
 //     periodic Cahn-Hilliard two steps per pass), one launch per member and
-//     pass, on a second compute stream, so they overlap the batch launches,
-//     and half of those run on a third between a fork and a join (all streams
-//     at the default priority). A round is planned on the host
-//     and queued on the
-//     compute stream; up to two rounds are queued ahead, so the device does
-//     not wait for the host between rounds;
+//     pass, on a second compute stream, so they overlap the batch launches;
+//     in a round without them half of the batch launches run there, between a
+//     fork and a join (both streams at the default priority). A round is planned
+//     on the host and queued on the compute stream; up to two rounds are queued
+//     ahead, so the device does not wait for the host between rounds;
 //   * when a request's last round is queued, the downloader waits for that
 //     round, takes the FP64 mass of the final state, copies it out and frees
 //     its buffers; only then is its memory counted free for admission.
@@ -123,8 +122,8 @@ struct mmspx_server {
 	int64_t next_id = 1;
 	std::chrono::steady_clock::time_point t0;
 	hipStream_t st = nullptr;   // compute (worker): batch launches
-	hipStream_t st2 = nullptr;  // compute (worker): the large members' single-grid launches
-	hipStream_t st3 = nullptr;  // compute (worker): half of a round's batch launches, between fork and join
+	hipStream_t st2 = nullptr;  // compute (worker): the large members' single-grid launches, or, in a round without them,
+	                            // half of the batch launches, between fork and join
 	hipEvent_t fork = nullptr, join = nullptr;
 	hipStream_t ust = nullptr;  // uploads
 	hipStream_t dst = nullptr;  // downloads
@@ -379,21 +378,25 @@ static int enqueue_round(mmspx_server* sv)
 	MMSPX_HIP(hipMemcpyAsync(sl.d_mem, sl.h_mem, sizeof(BMember) * act.size(), hipMemcpyHostToDevice, sv->st));
 	MMSPX_HIP(hipMemcpyAsync(sl.d_items, sl.h_items, sizeof(BItem) * (size_t)total, hipMemcpyHostToDevice, sv->st));
 	// The chains of launches (one per form and dimension) are independent, and a
-	// chain of small members leaves most of the GPU idle: the 3-D members of one
-	// form and the 2-D ones of the other run on a second stream, which starts
-	// behind the work lists' copies and which the compute stream waits for, so
-	// whatever is queued behind the round sees all of it done (16 requests of 21^3
-	// to 125^3 and 70^2 to 293^2 nodes: 15.7 ms on one stream, 12.6 on two)
-	const bool forked = (n2[0] > 0 || n3[1] > 0) && (n3[0] > 0 || n2[1] > 0);
+	// chain of small members leaves most of the GPU idle: in a round without large
+	// members the 3-D members of one form and the 2-D ones of the other run on the
+	// second stream, which starts behind the work lists' copies and which the
+	// compute stream waits for, so whatever is queued behind the round sees all of
+	// it done. Large members fill the GPU, and that stream, themselves. 16 requests
+	// of 21^3 to 125^3 and 70^2 to 293^2 nodes: 15.7 ms on one stream, 12.0 to
+	// 12.4 on two; with a stream of its own for the half, 12.6 to 15.2, by how many
+	// of the process's other streams share the four hardware queues with it
+	const bool solos = std::any_of(act.begin(), act.end(), [](const Request* r) { return r->solo; });
+	const bool forked = !solos && (n2[0] > 0 || n3[1] > 0) && (n3[0] > 0 || n2[1] > 0);
 	if (forked) {
 		MMSPX_HIP(hipEventRecord(sv->fork, sv->st));
-		MMSPX_HIP(hipStreamWaitEvent(sv->st3, sv->fork, 0));
+		MMSPX_HIP(hipStreamWaitEvent(sv->st2, sv->fork, 0));
 	}
 	int64_t launches = 0;
 	int passes[2][2];  // by group and dimension
 	for (int grp = 0; grp < 2; grp++) {
 		for (int dim = 2; dim <= 3; dim++) {
-			const hipStream_t st = forked && (grp == 1) == (dim == 3) ? sv->st3 : sv->st;
+			const hipStream_t st = forked && (grp == 1) == (dim == 3) ? sv->st2 : sv->st;
 			const int n = dim == 2 ? n2[grp] : n3[grp], spp = batch_steps_per_pass(sv->cfg.model, tile[grp], dim);
 			const BItem* it = sl.d_items + off[grp] + (dim == 2 ? 0 : n2[grp]);
 			passes[grp][dim - 2] = (steps + spp - 1) / spp;
@@ -405,7 +408,7 @@ static int enqueue_round(mmspx_server* sv)
 		}
 	}
 	if (forked) {
-		MMSPX_HIP(hipEventRecord(sv->join, sv->st3));
+		MMSPX_HIP(hipEventRecord(sv->join, sv->st2));
 		MMSPX_HIP(hipStreamWaitEvent(sv->st, sv->join, 0));
 	}
 	for (Request* r : act)
@@ -428,7 +431,7 @@ static int enqueue_round(mmspx_server* sv)
 	rd.steps = steps;
 	MMSPX_HIP(hipEventCreateWithFlags(&rd.ev, hipEventDisableTiming));
 	MMSPX_HIP(hipEventRecord(rd.ev, sv->st));
-	if (std::any_of(act.begin(), act.end(), [](const Request* r) { return r->solo; })) {
+	if (solos) {
 		MMSPX_HIP(hipEventCreateWithFlags(&rd.ev2, hipEventDisableTiming));
 		MMSPX_HIP(hipEventRecord(rd.ev2, sv->st2));
 	}
@@ -598,7 +601,6 @@ static void worker_main(mmspx_server* sv)
 		if (rc == 0) continue;
 		(void)hipStreamSynchronize(sv->st);
 		(void)hipStreamSynchronize(sv->st2);
-		(void)hipStreamSynchronize(sv->st3);
 		if (rc == 1) break;
 		// a device error: fail every request not yet finished and stop serving
 		std::lock_guard<std::mutex> lk(sv->mu);
@@ -633,7 +635,6 @@ int mmspx_server_create(const mmspx_server_config* cfg, mmspx_server** out)
 	int rc = 0;
 	if (hipGetDevice(&sv->device) != hipSuccess || hipStreamCreateWithFlags(&sv->st, hipStreamNonBlocking) != hipSuccess ||
 	    hipStreamCreateWithFlags(&sv->st2, hipStreamNonBlocking) != hipSuccess ||
-	    hipStreamCreateWithFlags(&sv->st3, hipStreamNonBlocking) != hipSuccess ||
 	    hipEventCreateWithFlags(&sv->fork, hipEventDisableTiming) != hipSuccess ||
 	    hipEventCreateWithFlags(&sv->join, hipEventDisableTiming) != hipSuccess ||
 	    hipStreamCreateWithFlags(&sv->ust, hipStreamNonBlocking) != hipSuccess ||
@@ -665,7 +666,6 @@ int mmspx_server_create(const mmspx_server_config* cfg, mmspx_server** out)
 		if (sv->pool) (void)hipMemPoolDestroy(sv->pool);
 		if (sv->st) (void)hipStreamDestroy(sv->st);
 		if (sv->st2) (void)hipStreamDestroy(sv->st2);
-		if (sv->st3) (void)hipStreamDestroy(sv->st3);
 		if (sv->fork) (void)hipEventDestroy(sv->fork);
 		if (sv->join) (void)hipEventDestroy(sv->join);
 		if (sv->ust) (void)hipStreamDestroy(sv->ust);
@@ -696,7 +696,6 @@ void mmspx_server_destroy(mmspx_server* sv)
 	if (sv->downloader.joinable()) sv->downloader.join();
 	(void)hipStreamSynchronize(sv->st);
 	(void)hipStreamSynchronize(sv->st2);
-	(void)hipStreamSynchronize(sv->st3);
 	(void)hipStreamSynchronize(sv->ust);
 	(void)hipStreamSynchronize(sv->dst);
 	std::set<Request*> fetched;  // fetched, still listed by rounds never retired
@@ -726,7 +725,6 @@ void mmspx_server_destroy(mmspx_server* sv)
 	(void)hipMemPoolDestroy(sv->pool);
 	(void)hipStreamDestroy(sv->st);
 	(void)hipStreamDestroy(sv->st2);
-	(void)hipStreamDestroy(sv->st3);
 	(void)hipEventDestroy(sv->fork);
 	(void)hipEventDestroy(sv->join);
 	(void)hipStreamDestroy(sv->ust);
