@@ -709,7 +709,7 @@ def main():
     dev_s, launches = g.step_timed(w["model"], w["params"], K)
     wall_s = time.perf_counter() - t0
     m1 = g.mass()
-    tile = g.get_tile()  # what the timed steps ran
+    tile = g.get_kernel()  # what the timed steps ran
     state = g.download()
     finite = bool(np.all(np.isfinite(state)))
     err64 = None
@@ -745,10 +745,10 @@ def main():
             "gg_aniso": "gga"}[w["model"]]
     if tile["variant"] != 2:
         kname = base + "_generic"
-    elif len(shape) == 3 and base == "gg" and tile["tz"] in (56, 58, 60):
+    elif tile["opt"] == 17:
         kname = "fmarch"
-    elif len(shape) == 3 and tile["tz"] == 56:
-        kname = "wmarch4"
+    elif tile["opt"] == 15:
+        kname = "wmarch4" if tile["tz"] == 56 else "march4"
     elif len(shape) == 3 and tile["opt"] == 8:
         kname = "march3d"
     elif len(shape) == 3 and tile["opt"] == 12:

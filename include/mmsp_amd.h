@@ -302,6 +302,12 @@ int mmspx_set_tile_options(mmspx_state* s, int body);
  * march). Before any tile is
  * set, reports what the last step ran (the Cahn-Hilliard default before any step). */
 int mmspx_get_tile(const mmspx_state* s, int* ty, int* tz, int* chunk);
+/* The same numbers for the kernel that the last mmspx_step ran its first pass
+ * on (before any step: the tile set, or the Cahn-Hilliard default), with that
+ * kernel's own body: 15 and 17 where mmspx_get_tile reports the body a default
+ * stands for. Set again with mmspx_set_tile and mmspx_set_tile_options, they
+ * run that kernel. */
+int mmspx_get_kernel(const mmspx_state* s, int* ty, int* tz, int* chunk);
 /* Project autotuner: times every candidate tile for `model` on this state's
  * shape (trial_steps each, state restored afterwards), keeps the fastest and
  * writes a one-line-per-candidate report. */

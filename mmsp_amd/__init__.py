@@ -117,6 +117,7 @@ def _load():
         "mmspx_set_variant": (C.c_int, [vp, C.c_int]),
         "mmspx_set_tile": (C.c_int, [vp, C.c_int, C.c_int, C.c_int]),
         "mmspx_get_tile": (C.c_int, [vp, P(C.c_int), P(C.c_int), P(C.c_int)]),
+        "mmspx_get_kernel": (C.c_int, [vp, P(C.c_int), P(C.c_int), P(C.c_int)]),
         "mmspx_set_tile_options": (C.c_int, [vp, C.c_int]),
         "mmspx_autotune": (C.c_int, [vp, C.c_int, dp, C.c_int, C.c_int, C.c_char_p, C.c_size_t]),
         "mmspx_kernel_time": (C.c_int, [vp, C.c_int, dp, C.c_int, C.c_int, dp, dp]),
@@ -329,10 +330,20 @@ class Grid:
         Zener pinning and 17 their 3-D field march (periodic)."""
         check(lib.mmspx_set_tile_options(self._h, int(body) if body is not None else (1 if register_queues else 0)))
 
-    def get_tile(self):
+    def _tile(self, get):
         ty, tz, ch = C.c_int(), C.c_int(), C.c_int()
-        v = lib.mmspx_get_tile(self._h, C.byref(ty), C.byref(tz), C.byref(ch))
+        v = get(self._h, C.byref(ty), C.byref(tz), C.byref(ch))
         return dict(variant=v % 16, ty=ty.value, tz=tz.value, chunk=ch.value, opt=v // 16)
+
+    def get_tile(self):
+        """The tile set, or the last step's; a default that runs body 15 or 17
+        reports the body of the pass it stands for (mmspx_get_tile)."""
+        return self._tile(lib.mmspx_get_tile)
+
+    def get_kernel(self):
+        """The kernel the last step ran its first pass on, with its own body
+        (mmspx_get_kernel)."""
+        return self._tile(lib.mmspx_get_kernel)
 
     def autotune(self, model, params, trial_steps=20):
         m = _model(model)

@@ -376,7 +376,7 @@ static int step_impl(mmspx_state* s, int model, const double* params, int np, in
 	} else if (s->variant == 2) {
 		return fail(MMSPX_EUNSUPPORTED, "no tiled/fused kernel for this model, shape and boundary condition");
 	}
-	s->last = fused ? tc : TuneChoice{1, 0, 0, 0, 0};
+	s->last = s->ran = fused ? tc : TuneChoice{1, 0, 0, 0, 0};
 	if (s->last.opt == 15) s->last.opt = march4_reported_body(g, model);
 	if (s->last.opt == 17) s->last.opt = one_step_choice(g, s->desc.precision, model).opt;
 	s->has_last = true;
@@ -562,6 +562,16 @@ int mmspx_get_tile(const mmspx_state* s, int* ty, int* tz, int* chunk)
 	if (!s) return fail(MMSPX_EINVAL, "null state");
 	TuneChoice t = s->tuned ? s->tile : s->has_last ? s->last : default_choice(s->geom, s->desc.precision, MMSPX_CH_DW);
 	if (!s->tuned && t.opt == 15) t.opt = march4_reported_body(s->geom, MMSPX_CH_DW);
+	if (ty) *ty = t.ty;
+	if (tz) *tz = t.tz;
+	if (chunk) *chunk = t.chunk;
+	return t.variant + 16 * t.opt;
+}
+
+int mmspx_get_kernel(const mmspx_state* s, int* ty, int* tz, int* chunk)
+{
+	if (!s) return fail(MMSPX_EINVAL, "null state");
+	const TuneChoice t = s->has_last ? s->ran : s->tuned ? s->tile : default_choice(s->geom, s->desc.precision, MMSPX_CH_DW);
 	if (ty) *ty = t.ty;
 	if (tz) *tz = t.tz;
 	if (chunk) *chunk = t.chunk;

@@ -106,6 +106,7 @@ struct mmspx_state {
 	bool tuned = false;      // a tile chosen by mmspx_set_tile / mmspx_autotune
 	mmspx::TuneChoice tile{};
 	mmspx::TuneChoice last{};  // what the last step ran (reported by mmspx_get_tile when not tuned)
+	mmspx::TuneChoice ran{};   // the kernel the last step's first pass ran (mmspx_get_kernel)
 	bool has_last = false;
 	int64_t launches = 0;
 	int64_t steps_run = 0;
