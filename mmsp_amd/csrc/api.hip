@@ -376,7 +376,9 @@ static int step_impl(mmspx_state* s, int model, const double* params, int np, in
 	} else if (s->variant == 2) {
 		return fail(MMSPX_EUNSUPPORTED, "no tiled/fused kernel for this model, shape and boundary condition");
 	}
-	s->last = s->ran = fused ? tc : TuneChoice{1, 0, 0, 0, 0};
+	// a default's calls end in the passes their last steps are fastest on
+	auto pass = [&](int left) { return fused && !s->tuned ? pass_choice(g, s->desc.precision, model, tc, left) : tc; };
+	s->last = s->ran = fused ? pass(steps) : TuneChoice{1, 0, 0, 0, 0};
 	if (s->last.opt == 15) s->last.opt = march4_reported_body(g, model);
 	if (s->last.opt == 17) s->last.opt = one_step_choice(g, s->desc.precision, model).opt;
 	s->has_last = true;
@@ -437,9 +439,10 @@ static int step_impl(mmspx_state* s, int model, const double* params, int np, in
 		}
 	}
 	while (steps > 0) {
-		const int n = std::min(steps, spl);
+		const TuneChoice t = pass(steps);
+		const int n = std::min(steps, fused ? fused_steps_per_launch(model, t) : 1);
 		p.step = (uint64_t)s->steps_run;
-		rc = fused ? launch_fused_step(g, s->desc.precision, p, s->cur, s->nxt, s->stream, tc, n, &s->launches, s->aux)
+		rc = fused ? launch_fused_step(g, s->desc.precision, p, s->cur, s->nxt, s->stream, t, n, &s->launches, s->aux)
 		           : launch_generic_step(g, s->desc.precision, p, s->cur, s->nxt, s->aux, s->stream, &s->launches);
 		if (rc) return rc;
 		std::swap(s->cur, s->nxt);

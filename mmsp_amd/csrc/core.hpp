@@ -154,6 +154,9 @@ int fused_steps_per_launch(int model, const TuneChoice& t);
 TuneChoice default_choice(const Geom& g, int prec, int model);
 // the default without the 2-D multi-step wave strips and the four-level march
 TuneChoice one_step_choice(const Geom& g, int prec, int model);
+// the kernel of a call's next pass where `left` steps remain and the call runs
+// the default `full`
+TuneChoice pass_choice(const Geom& g, int prec, int model, const TuneChoice& full, int left);
 int launch_reduce(const Geom& g, int prec, int what, const ModelParams& p, const void* a, double* part,
                   hipStream_t st);
 int launch_transpose(const void* src, void* dst, int nodes, int fields, size_t elem, bool to_field_major,
@@ -176,6 +179,7 @@ bool march4_tile_known(int prec, int ty, int tz);
 bool march4_choice(const Geom& g, int prec, int model, TuneChoice* out);
 TuneChoice march4_choice_many(const Geom* const* g, int count, int prec);  // one launch over all of them
 int march4_reported_body(const Geom& g, int model);
+bool march4_last_step_choice(const Geom& g, int prec, const TuneChoice& full, TuneChoice* out);
 int launch_march4(const Geom& g, int prec, const ModelParams& p, const void* a, void* b, hipStream_t st,
                   const TuneChoice& t, int nsteps);
 // 2-D multi-phase grain growth, wave strips (kernels_gga2d.hip)

@@ -365,13 +365,36 @@ static TuneChoice two_step_choice(const Geom& g, int prec)
 // FP32 5.6 (7.1). 128^3 x 8 FP32 gains nothing (29.5 against 28.6), and 8 FP64
 // fields fit the LDS on 8 x 32 tiles only (256^3: 488.5 against 481.0): those
 // stay on the one-step march.
+// Allen-Cahn (the last two steps of a call, pass_choice): 16 x 64 or 32 x 64
+// tiles and the chunk from the cost model of two_step_choice: rounds x (chunk +
+// 3 planes) x owned points per thread (16 x 64: 1188 on 640 threads, two
+// workgroups per CU in rounds of 512 each 1.7 times as long; 32 x 64: 2244 on
+// 768, one per CU).
 static bool march2_choice(const Geom& g, int prec, int model, TuneChoice* out)
 {
 	constexpr int kCUs = 256;
 	if (!all_periodic(g) || (prec != MMSPX_F64 && prec != MMSPX_F32)) return false;
-	if (model != MMSPX_GG && model != MMSPX_ZENER) return false;
+	if (model != MMSPX_AC && model != MMSPX_GG && model != MMSPX_ZENER) return false;
 	const int nz = g.n[2], pad = (nz + 63) / 64 * 64 - nz;
 	if (pad * 8 > nz) return false;
+	if (model == MMSPX_AC) {
+		double best_cost = 1e300;
+		for (int ty : {16, 32}) {
+			const double own = ty == 16 ? 1188.0 / 640 : 2244.0 / 768;
+			const int64_t tiles = (int64_t)((g.n[1] + ty - 1) / ty) * ((nz + 63) / 64);
+			for (int c : {4, 8, 16, 32, 64}) {
+				const int64_t wgs = tiles * ((g.n[0] + c - 1) / c);
+				const double rounds = (ty == 16 && wgs > kCUs) ? 1.7 * (double)((wgs + 2 * kCUs - 1) / (2 * kCUs))
+				                                               : (double)((wgs + kCUs - 1) / kCUs);
+				const double cost = rounds * (c + 3) * own;
+				if (cost < best_cost) {
+					best_cost = cost;
+					*out = TuneChoice{2, ty, 64, c, 12};
+				}
+			}
+		}
+		return true;
+	}
 	const int q = g.fields;
 	if (!(q == 2 || q == 4 || (q == 8 && prec == MMSPX_F32 && g.nodes >= ((int64_t)1 << 22)))) return false;
 	const int per_cu = q == 2 ? 2 : 1;
@@ -390,6 +413,65 @@ TuneChoice default_choice(const Geom& g, int prec, int model)
 	if (fmarch_choice(g, prec, model, &t)) return t;
 	if (march4_choice(g, prec, model, &t)) return t;
 	return one_step_choice(g, prec, model);
+}
+
+// A multi-step pass cut short forms fewer levels on tiles made for all of them,
+// so the steps left over at a call's end, and calls of fewer steps than a pass,
+// go to a one- or two-step kernel where that takes less (us a call, cut pass and
+// this):
+// - 2-D periodic Allen-Cahn up to 2^20 nodes: temporal blocks, which take up to
+//   eight steps in one launch: FP64 128^2 6 steps 8.6 and 6.0, 512^2 14.0 and 9.1
+//   for 7, 1024^2 9.6 and 7.9 for one; four are a whole pass of four levels.
+//   From 1300^2 the strips are faster throughout (one step 9.8 and 11.8).
+// - one step of 2-D Allen-Cahn between walls, and two between 2^20 and 2^23
+//   nodes: the wave strips (FP64 1024^2 8.7 and 5.6; FP32 2048^2 15.7 and 8.9,
+//   two steps 19.5 and 17.1; two at 700^2 7.1 and 8.6, at 4096^2 42 and 45).
+// - one step of 2-D Cahn-Hilliard: its wave strips (1024^2 FP64 8.4 and 6.5,
+//   FP32 7.3 and 5.7; 2048^2 FP32 14.6 and 10.1).
+// - one or two steps of 2-D grain growth and Zener pinning: the split strips
+//   (512^2 x 32 FP32 one 21.2 and 16.4, two 29.3 and 22.9).
+// - one step of 3-D Allen-Cahn: the plane march (FP64 64^3 10.2 and 5.8, 256^3
+//   69 and 45; FP32 41 and 24); two, from 2^20 nodes: that march two steps per
+//   pass where it fits (256^3 FP64 73 and 60, FP32 42 and 35).
+// - one step of 3-D Cahn-Hilliard: march4_last_step_choice.
+// - one step of 3-D grain growth and Zener pinning: the plane march (192^3 x 8
+//   FP32 157 and 120, 256^3 x 8 392 and 243, 96^3 x 4 16.4 and 11.9), but for 8
+//   fields in FP64 where its 64-node tile rows would be padded by more than an
+//   eighth (150 x 203 x 97 130 and 152, 96^3 34 and 39).
+TuneChoice pass_choice(const Geom& g, int prec, int model, const TuneChoice& full, int left)
+{
+	if (full.opt < 13 || full.opt > 17) return full;
+	const int64_t nodes = g.nodes;
+	if (g.dim == 2 && model == MMSPX_AC && all_periodic(g)) {
+		const bool blocks = left < kTbMaxSteps && left != 4 && nodes <= ((int64_t)1 << 20);
+		return blocks ? one_step_choice(g, prec, model) : full;
+	}
+	if (left >= fused_steps_per_launch(model, full)) return full;
+	TuneChoice t = full;
+	switch (full.opt) {
+	case 13:
+	case 14:
+		if (left == 1 || (left == 2 && model == MMSPX_AC && nodes >= ((int64_t)1 << 20) && nodes < ((int64_t)1 << 23)))
+			t = one_step_choice(g, prec, model);
+		break;
+	case 15:
+		if (model == MMSPX_AC) {
+			if (left == 1) t = one_step_choice(g, prec, model);
+			else if (left == 2 && nodes >= ((int64_t)1 << 20) && !march2_choice(g, prec, model, &t)) t = full;
+		} else if (!march4_last_step_choice(g, prec, full, &t)) {
+			t = full;
+		}
+		break;
+	case 16:
+		if (left <= 2) t = one_step_choice(g, prec, model);
+		break;
+	case 17: {
+		const int pad = (g.n[2] + 63) / 64 * 64 - g.n[2];
+		if (left == 1 && !(g.fields == 8 && prec == MMSPX_F64 && pad * 8 > g.n[2])) t = one_step_choice(g, prec, model);
+		break;
+	}
+	}
+	return t.variant == 2 ? t : full;
 }
 
 // Defaults come from sweeps of the candidates below on MI355X (the figures
@@ -449,7 +531,7 @@ TuneChoice one_step_choice(const Geom& g, int prec, int model)
 		return TuneChoice{2, 8, 64, chunk, 8};
 	}
 	TuneChoice two;
-	if (g.dim == 3 && march2_choice(g, prec, model, &two)) return two;
+	if (g.dim == 3 && model != MMSPX_AC && march2_choice(g, prec, model, &two)) return two;
 	if (g.dim == 3 && (model == MMSPX_AC || model == MMSPX_AC_NOISE || model == MMSPX_GG || model == MMSPX_ZENER)) {
 		const bool scalar = model == MMSPX_AC || model == MMSPX_AC_NOISE;
 		const int ty = scalar ? (prec == MMSPX_F64 ? 16 : 32) : 8;

@@ -62,11 +62,12 @@ static int64_t march_wgs(const Geom& g, int ty, int tz, int c)
 	return (int64_t)((g.n[1] + ty - 1) / ty) * ((g.n[2] + tz - 1) / tz) * ((g.n[0] + c - 1) / c);
 }
 
+static const double tau[2][7][6] = {
+    {{1.45}, {1.36}, {1.36}, {1.00, 1.51}, {0.92, 1.10, 1.30, 1.51}, {1.30}, {1.94}},
+    {{1.31}, {1.08, 1.64}, {1.05, 1.41}, {0.79, 1.00, 1.26, 1.52}, {0.77, 0.86, 0.96, 1.06, 1.16, 1.26}, {0.97, 1.39}, {1.10, 1.62}}};
+
 static TuneChoice march_best(const Geom* const* g, int count, int prec, int model, int tiles)
 {
-	static const double tau[2][7][6] = {
-	    {{1.45}, {1.36}, {1.36}, {1.00, 1.51}, {0.92, 1.10, 1.30, 1.51}, {1.30}, {1.94}},
-	    {{1.31}, {1.08, 1.64}, {1.05, 1.41}, {0.79, 1.00, 1.26, 1.52}, {0.77, 0.86, 0.96, 1.06, 1.16, 1.26}, {0.97, 1.39}, {1.10, 1.62}}};
 	const int f = prec == MMSPX_F64 ? 0 : 1;
 	TuneChoice out{2, 16, 32, 8, 15};
 	double us = 1e300;
@@ -107,6 +108,28 @@ int launch_march4(const Geom& g, int prec, const ModelParams& p, const void* a, 
 	if (t.chunk < 1 || nsteps < 1) return fail(MMSPX_EINVAL, "bad chunk or step count");
 	return prec == MMSPX_F64 ? launch_march4_prec<MMSPX_F64>(g, p, a, b, st, t, nsteps)
 	                         : launch_march4_f32(g, p, a, b, st, t, nsteps);
+}
+
+// A last single Cahn-Hilliard step: the march's short pass (two of its levels;
+// 0.84 of a whole pass in FP64, 0.92 in FP32) or body 2, the register queues on
+// 32 x 64 tiles, which run in rounds of one workgroup a CU in FP64, of two in
+// FP32. us, short pass and body 2: FP64 192^3 33 and 48, 224^3 43 and 51, 240^3
+// 54 and 53, 256^3 66 and 59, 320^3 131 and 145; FP32 176^3 22 and 21, 192^3 25
+// and 22, 224^3 30 and 32, 256^3 44 and 36, 320^3 77 and 65.
+bool march4_last_step_choice(const Geom& g, int prec, const TuneChoice& full, TuneChoice* out)
+{
+	const int f = prec == MMSPX_F64 ? 0 : 1;
+	int k = 0;
+	while (k < 6 && !(kTiles[f][k][0] == full.ty && kTiles[f][k][1] == full.tz)) k++;
+	const double march = (f ? 0.92 : 0.84) * march_time(march_wgs(g, full.ty, full.tz, full.chunk), full.chunk, tau[f][k]);
+	*out = TuneChoice{2, 32, 64, f ? 16 : 32, 2};
+	// fitted to the figures above: a round of w workgroups
+	auto round_us = [&](double w) {
+		return w <= 0.0 ? 0.0 : f == 0 ? 47.0 + 12.5 * w / 256.0 : w <= 256.0 ? 21.0 + 1.5 * w / 256.0 : 22.0 + 14.0 * w / 512.0;
+	};
+	const int64_t wgs = march_wgs(g, out->ty, out->tz, out->chunk), full_round = f ? 512 : 256;
+	const double queues = (double)(wgs / full_round) * round_us((double)full_round) + round_us((double)(wgs % full_round));
+	return queues < march;
 }
 
 // The body mmspx_get_tile reports for a default the four-level march runs: the

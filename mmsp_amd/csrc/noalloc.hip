@@ -88,14 +88,14 @@ extern "C" int mmspx_step_noalloc(const mmspx_desc* desc, void* buf0, void* buf1
 		                              std::to_string((size_t)MMSPX_NOALLOC_SCRATCH_BYTES) +
 		                              " bytes (use mmspx_step on a state)");
 	hipStream_t st = (hipStream_t)stream;
-	const int spl = fused ? fused_steps_per_launch(model, tc) : 1;
 	void *a = buf0, *b = buf1;
 	int which = 0;
 	int64_t launches = 0, done = 0;
 	while (steps > 0) {
-		const int n = std::min(steps, spl);
+		const TuneChoice t = fused ? pass_choice(g, desc->precision, model, tc, steps) : tc;
+		const int n = std::min(steps, fused ? fused_steps_per_launch(model, t) : 1);
 		p.step = (uint64_t)(first_step + done);
-		rc = fused ? launch_fused_step(g, desc->precision, p, a, b, st, tc, n, &launches, needs_plane ? sp : nullptr)
+		rc = fused ? launch_fused_step(g, desc->precision, p, a, b, st, t, n, &launches, needs_plane ? sp : nullptr)
 		           : launch_generic_step(g, desc->precision, p, a, b, needs_plane ? sp : nullptr, st, &launches);
 		if (rc) return rc;
 		std::swap(a, b);

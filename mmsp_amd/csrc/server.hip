@@ -416,12 +416,12 @@ static int enqueue_round(mmspx_server* sv)
 	// the large 3-D members: their own single-grid launches
 	for (Request* r : act) {
 		if (!r->solo) continue;
-		const int spl = fused_steps_per_launch(sv->cfg.model, r->tile);
 		for (int left = steps; left > 0;) {
-			const int n = std::min(left, spl);
+			const TuneChoice t = pass_choice(r->g, r->prec, sv->cfg.model, r->tile, left);
+			const int n = std::min(left, fused_steps_per_launch(sv->cfg.model, t));
 			const char* a = r->dev + (r->cur ? r->bytes : 0);
 			char* b = r->dev + (r->cur ? 0 : r->bytes);
-			rc = launch_fused_step(r->g, r->prec, r->p, a, b, sv->st2, r->tile, n, &launches);
+			rc = launch_fused_step(r->g, r->prec, r->p, a, b, sv->st2, t, n, &launches);
 			if (rc) return rc;
 			r->cur ^= 1;
 			left -= n;
