@@ -348,8 +348,8 @@ class Grid:
     def autotune(self, model, params, trial_steps=20):
         m = _model(model)
         p = _params(m, params)
-        buf = C.create_string_buffer(8192)
-        check(lib.mmspx_autotune(self._h, m, _dp(p), p.size, int(trial_steps), buf, 8192))
+        buf = C.create_string_buffer(16384)
+        check(lib.mmspx_autotune(self._h, m, _dp(p), p.size, int(trial_steps), buf, 16384))
         return buf.value.decode()
 
     def kernel_time(self, model, params, reps):

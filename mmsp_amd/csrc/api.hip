@@ -637,8 +637,11 @@ int mmspx_autotune(mmspx_state* s, int model, const double* params, int np, int 
 	int rc = make_params(model, params, np, &p);
 	if (rc) return rc;
 	std::string rep;
-	TuneChoice cand[96];
-	int nc = fused_supported(s->geom, s->desc.precision, model) ? tile_candidates(s->geom, s->desc.precision, model, cand, 96) : 0;
+	constexpr int kCandidates = 128;
+	TuneChoice cand[kCandidates];
+	int nc = fused_supported(s->geom, s->desc.precision, model)
+	             ? tile_candidates(s->geom, s->desc.precision, model, cand, kCandidates)
+	             : 0;
 	// keep the state: every trial starts from it and it is restored at the end
 	void* saved = nullptr;
 	if (hipMalloc(&saved, s->bytes) != hipSuccess) return fail(MMSPX_ENOMEM, "device allocation failed");

@@ -177,6 +177,7 @@ bool march4_supported(const Geom& g, int prec, int model);
 int march4_max_steps(int model);
 bool march4_tile_known(int prec, int ty, int tz);
 bool march4_choice(const Geom& g, int prec, int model, TuneChoice* out);
+int march4_candidates(const Geom& g, int prec, int model, TuneChoice* out, int max);
 TuneChoice march4_choice_many(const Geom* const* g, int count, int prec);  // one launch over all of them
 int march4_reported_body(const Geom& g, int model);
 bool march4_last_step_choice(const Geom& g, int prec, const TuneChoice& full, TuneChoice* out);

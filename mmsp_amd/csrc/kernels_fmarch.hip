@@ -124,9 +124,12 @@ int fmarch_candidates(const Geom& g, int prec, int model, TuneChoice* out, int m
 	int n = 0;
 	if (!fmarch_supported(g, prec, model)) return 0;
 	for (const FieldTile& t : kFieldTiles)
-		if (t.prec == prec && t.fields == g.fields)
-			for (int c : {4, 8, 16, 32, 64})
+		if (t.prec == prec && t.fields == g.fields) {
+			TuneChoice best;
+			best_pass(g, t, &best);
+			for (int c : {best.chunk, 4, 8, 16, 32, 64})
 				if (n < max) out[n++] = TuneChoice{2, t.ty, t.tz, c, 17};
+		}
 	return n;
 }
 

@@ -688,6 +688,12 @@ int tile_candidates(const Geom& g, int prec, int model, TuneChoice* out, int max
 		if (n < max) out[n++] = TuneChoice{2, ty, tz, chunk, opt};
 	};
 	const bool ch = ch_family(model);
+	// the default itself (its tile and chunk come from a cost model, not from the
+	// lists below), so that tuning never ends on a slower one
+	const TuneChoice def = default_choice(g, prec, model);
+	if (def.variant == 2) add(def.ty, def.tz, def.chunk, def.opt);
+	// Allen-Cahn and Cahn-Hilliard, 3-D periodic: the four-level march
+	n += march4_candidates(g, prec, model, out + n, max - n);
 	// grain growth and Zener pinning, periodic: several steps per pass
 	n += fmarch_candidates(g, prec, model, out + n, max - n);
 	if (fields2d_supported(g, prec, model))
@@ -730,9 +736,6 @@ int tile_candidates(const Geom& g, int prec, int model, TuneChoice* out, int max
 		// (Ostwald ripening: the one-pass march)
 		const bool two = all_periodic(g) && model != MMSPX_AC_NOISE && model != MMSPX_GG_ANISO &&
 		                 (prec == MMSPX_F64 || prec == MMSPX_F32);
-		if (march4_supported(g, prec, model))
-			for (int c : {4, 8, 16, 32, 64})
-				for (auto& t : {std::pair<int, int>{26, 52}, {32, 32}, {16, 32}, {16, 16}}) add(t.first, t.second, c, 15);
 		if (two)
 			for (int c : {8, 16, 32, 64}) {
 				if (scalar) {
@@ -761,10 +764,6 @@ int tile_candidates(const Geom& g, int prec, int model, TuneChoice* out, int max
 		// two steps per pass (deterministic chemical potentials, periodic grids)
 		if ((model == MMSPX_CH || model == MMSPX_CH_DW) && !edges)
 			for (int c : {6, 8, 12, 16, 24, 32, 48, 64}) {
-				if (march4_supported(g, prec, model) && c != 6 && c != 12) {
-					add(26, 52, c, 15);
-					add(16, 32, c, 15);
-				}
 				add(32, 64, c, 6);
 				add(32, 32, c, 7);
 			}

@@ -66,24 +66,52 @@ static const double tau[2][7][6] = {
     {{1.45}, {1.36}, {1.36}, {1.00, 1.51}, {0.92, 1.10, 1.30, 1.51}, {1.30}, {1.94}},
     {{1.31}, {1.08, 1.64}, {1.05, 1.41}, {0.79, 1.00, 1.26, 1.52}, {0.77, 0.86, 0.96, 1.06, 1.16, 1.26}, {0.97, 1.39}, {1.10, 1.62}}};
 
-static TuneChoice march_best(const Geom* const* g, int count, int prec, int model, int tiles)
+// the chunk of least time on tile k; us receives that time
+static TuneChoice march_best_chunk(const Geom* const* g, int count, int prec, int model, int k, double* us)
 {
-	const int f = prec == MMSPX_F64 ? 0 : 1;
-	TuneChoice out{2, 16, 32, 8, 15};
-	double us = 1e300;
-	for (int k = 0; k < tiles; k++) {
-		const int ty = kTiles[f][k][0], tz = kTiles[f][k][1];
-		for (int c = 3; c <= 64; c += count > 1 && c >= 8 ? 4 : 1) {
-			int64_t wgs = 0;
-			for (int m = 0; m < count; m++) wgs += march_wgs(*g[m], ty, tz, c);
-			const double t = march_time(wgs, c, tau[f][k]) * (k >= 5 && f == 1 && model == MMSPX_AC ? 1.09 : 1.0);
-			if (t < us) {
-				us = t;
-				out = TuneChoice{2, ty, tz, c, 15};
-			}
+	const int f = prec == MMSPX_F64 ? 0 : 1, ty = kTiles[f][k][0], tz = kTiles[f][k][1];
+	TuneChoice out{2, ty, tz, 8, 15};
+	*us = 1e300;
+	for (int c = 3; c <= 64; c += count > 1 && c >= 8 ? 4 : 1) {
+		int64_t wgs = 0;
+		for (int m = 0; m < count; m++) wgs += march_wgs(*g[m], ty, tz, c);
+		const double t = march_time(wgs, c, tau[f][k]) * (k >= 5 && f == 1 && model == MMSPX_AC ? 1.09 : 1.0);
+		if (t < *us) {
+			*us = t;
+			out.chunk = c;
 		}
 	}
 	return out;
+}
+
+static TuneChoice march_best(const Geom* const* g, int count, int prec, int model, int tiles)
+{
+	TuneChoice out{};
+	double us = 1e300;
+	for (int k = 0; k < tiles; k++) {
+		double t;
+		const TuneChoice c = march_best_chunk(g, count, prec, model, k, &t);
+		if (t < us) {
+			us = t;
+			out = c;
+		}
+	}
+	return out;
+}
+
+// every tile with the model's chunk, half of it and twice it
+int march4_candidates(const Geom& g, int prec, int model, TuneChoice* out, int max)
+{
+	int n = 0;
+	if (!march4_supported(g, prec, model)) return 0;
+	const Geom* one = &g;
+	for (int k = 0; k < 7; k++) {
+		double us;
+		const TuneChoice t = march_best_chunk(&one, 1, prec, model, k, &us);
+		for (int c : {t.chunk / 2, t.chunk, 2 * t.chunk})
+			if (c >= 2 && n < max) out[n++] = TuneChoice{2, t.ty, t.tz, c, 15};
+	}
+	return n;
 }
 
 TuneChoice march4_choice_many(const Geom* const* g, int count, int prec)
