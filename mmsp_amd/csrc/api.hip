@@ -354,6 +354,17 @@ static bool same_baked_params(const ModelParams& a, const ModelParams& b)
 	return true;
 }
 
+// The kernel of the state's steps of `model`: the tile set, or the default. A
+// tile the autotuner chose for another model gives way to the default where it
+// is a multi-step body that does not run this one.
+static TuneChoice choice_of(const mmspx_state* s, int model)
+{
+	if (s->tuned && (s->tuned_model < 0 || s->tuned_model == model ||
+	                 multi_step_body_runs(s->geom, s->desc.precision, model, s->tile.opt)))
+		return s->tile;
+	return default_choice(s->geom, s->desc.precision, model);
+}
+
 static int step_impl(mmspx_state* s, int model, const double* params, int np, int steps)
 {
 	if (!s) return fail(MMSPX_EINVAL, "null state");
@@ -367,7 +378,7 @@ static int step_impl(mmspx_state* s, int model, const double* params, int np, in
 	bool fused = false;
 	TuneChoice tc{};
 	if (s->variant != 1 && fused_supported(g, s->desc.precision, model)) {
-		tc = s->tuned ? s->tile : default_choice(g, s->desc.precision, model);
+		tc = choice_of(s, model);
 		if (s->variant == 2 && tc.variant != 2) tc = default_choice(g, s->desc.precision, model);
 		// where one thread per node is the default: the 3-D plane march, the 2-D strips
 		if (s->variant == 2 && tc.variant != 2)
@@ -376,8 +387,9 @@ static int step_impl(mmspx_state* s, int model, const double* params, int np, in
 	} else if (s->variant == 2) {
 		return fail(MMSPX_EUNSUPPORTED, "no tiled/fused kernel for this model, shape and boundary condition");
 	}
-	// a default's calls end in the passes their last steps are fastest on
-	auto pass = [&](int left) { return fused && !s->tuned ? pass_choice(g, s->desc.precision, model, tc, left) : tc; };
+	// calls end in the passes their last steps are fastest on, unless the caller set the tile
+	const bool set = s->tuned && s->tuned_model < 0;
+	auto pass = [&](int left) { return fused && !set ? pass_choice(g, s->desc.precision, model, tc, left) : tc; };
 	s->last = s->ran = fused ? pass(steps) : TuneChoice{1, 0, 0, 0, 0};
 	if (s->last.opt == 15) s->last.opt = march4_reported_body(g, model);
 	if (s->last.opt == 17) s->last.opt = one_step_choice(g, s->desc.precision, model).opt;
@@ -492,6 +504,7 @@ int mmspx_set_tile(mmspx_state* s, int ty, int tz, int chunk)
 	if (!tile_known(s->geom, t)) return fail(MMSPX_EINVAL, "no compiled tile of that shape for this grid");
 	s->tile = t;
 	s->tuned = true;
+	s->tuned_model = -1;
 	return 0;
 }
 
@@ -507,6 +520,7 @@ int mmspx_set_tile_options(mmspx_state* s, int body)
 		s->tile = one_step_choice(s->geom, s->desc.precision, MMSPX_CH_DW);
 		s->tuned = true;
 	}
+	s->tuned_model = -1;
 	s->tile.opt = body;
 	// 2-D: the split strips run 1 x 64 strips (bodies 4, 5), two steps per
 	// pass 1 x kChWaveOut (bodies 9, 10)
@@ -586,7 +600,7 @@ int mmspx_get_kernel(const mmspx_state* s, int* ty, int* tz, int* chunk)
 static int steps_per_launch_now(const mmspx_state* s, int model)
 {
 	if (s->variant == 1 || !fused_supported(s->geom, s->desc.precision, model)) return 1;
-	TuneChoice tc = s->tuned ? s->tile : default_choice(s->geom, s->desc.precision, model);
+	TuneChoice tc = choice_of(s, model);
 	if (s->variant == 2 && tc.variant != 2) tc = default_choice(s->geom, s->desc.precision, model);
 	return tc.variant == 2 ? fused_steps_per_launch(model, tc) : 1;
 }
@@ -648,7 +662,9 @@ int mmspx_autotune(mmspx_state* s, int model, const double* params, int np, int 
 	MMSPX_HIP(hipMemcpyAsync(saved, s->cur, s->bytes, hipMemcpyDeviceToDevice, s->stream));
 	const int old_variant = s->variant;
 	const bool old_tuned = s->tuned;
+	const int old_model = s->tuned_model;
 	const TuneChoice old_tile = s->tile;
+	s->tuned_model = -1;  // a trial runs its own tile
 	const int64_t old_steps = s->steps_run;  // the stochastic forms' noise continues from here
 	double best = 1e30;
 	TuneChoice best_t{1, 0, 0, 0, 0};
@@ -682,11 +698,13 @@ int mmspx_autotune(mmspx_state* s, int model, const double* params, int np, int 
 	s->steps_run = old_steps;
 	if (rc) {
 		s->tuned = old_tuned;
+		s->tuned_model = old_model;
 		s->tile = old_tile;
 		return rc;
 	}
 	s->tile = best_t;
 	s->tuned = true;
+	s->tuned_model = model;
 	if (report && report_len) {
 		std::snprintf(report, report_len, "%s", rep.c_str());
 	}

@@ -104,6 +104,7 @@ struct mmspx_state {
 	int device = 0;
 	int variant = 0;
 	bool tuned = false;      // a tile chosen by mmspx_set_tile / mmspx_autotune
+	int tuned_model = -1;    // the model mmspx_autotune chose it for
 	mmspx::TuneChoice tile{};
 	mmspx::TuneChoice last{};  // what the last step ran (reported by mmspx_get_tile when not tuned)
 	mmspx::TuneChoice ran{};   // the kernel the last step's first pass ran (mmspx_get_kernel)
@@ -171,6 +172,8 @@ int copy_to_device(void* dst, const void* src, size_t bytes, hipStream_t st);
 void staging_retain();
 void staging_release();
 bool tile_known(const Geom& g, const TuneChoice& t);
+// a multi-step body (13 to 17) runs this model on this grid; true for other bodies
+bool multi_step_body_runs(const Geom& g, int prec, int model, int body);
 // 3-D four-level march (kernels_march4.hip), tile body 15: two Cahn-Hilliard
 // or four Allen-Cahn steps per pass on periodic grids
 bool march4_supported(const Geom& g, int prec, int model);

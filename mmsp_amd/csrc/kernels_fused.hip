@@ -661,6 +661,18 @@ TuneChoice one_step_choice(const Geom& g, int prec, int model)
 	return TuneChoice{2, 32, 64, prec == MMSPX_F64 ? 32 : 16, 2};
 }
 
+bool multi_step_body_runs(const Geom& g, int prec, int model, int body)
+{
+	switch (body) {
+	case 13:
+	case 14: return steps2d_supported(g, prec, model);
+	case 15: return march4_supported(g, prec, model);
+	case 16: return fields2d_supported(g, prec, model);
+	case 17: return fmarch_supported(g, prec, model);
+	}
+	return true;
+}
+
 bool tile_known(const Geom& g, const TuneChoice& t)
 {
 	if (t.chunk < 2 || t.chunk > 4096) return false;
