@@ -292,7 +292,10 @@ int mmspx_set_tile(mmspx_state* s, int ty, int tz, int chunk);
  * growth and Zener pinning with 2, 4 or 8 fields in the same forms: 17 is the
  * field march, two to four steps per pass on tiles of 60, 58 or 56 columns
  * (their default where it is the fastest; a default reports the body it stands
- * for, 12 or 8). */
+ * for, 12 or 8). 13 to 15 are refused on vector grids, 16 and 17 on scalar ones
+ * and on field counts they are not compiled for; a body set after one of them
+ * leaves a tile that only they run for 1 x 64 (2-D), 32 x 64, or 8 x 64 on 3-D
+ * vector grids. */
 int mmspx_set_tile_options(mmspx_state* s, int body);
 /* Returns variant + 16 * tile body (1: register queues, or the 2-D
  * grain-growth tile; 2: wave strips, or 3-D register queues on 768 threads;

@@ -469,6 +469,17 @@ int mmspx_step(mmspx_state* s, int model, const double* params, int np, int step
 	return step_impl(s, model, params, np, steps);
 }
 
+// Bodies 13 to 15 run scalar grids, 16 and 17 vector grids of the field counts
+// they are compiled for.
+static bool body_takes_grid(const mmspx_state* s, int body)
+{
+	const int q = s->geom.fields;
+	if (body >= 13 && body <= 15) return !s->desc.vector;
+	if (body == 16) return s->desc.vector && (q == 2 || q == 4 || q == 8 || q == 16 || q == 32);
+	if (body == 17) return s->desc.vector && fmarch_any_tile(s->desc.precision, q, 0).ty > 0;
+	return true;
+}
+
 int mmspx_set_tile(mmspx_state* s, int ty, int tz, int chunk)
 {
 	if (!s) return fail(MMSPX_EINVAL, "null state");
@@ -483,23 +494,24 @@ int mmspx_set_tile(mmspx_state* s, int ty, int tz, int chunk)
 	if (s->geom.dim == 2 && ty > 1 && tz == kTbCols) opt = 3;
 	else if (s->geom.dim == 2 && ty > 1) opt = 1;
 	else if (s->geom.dim == 2 && s->tuned && s->tile.ty > 1) opt = 0;
-	// 1 x 48 and 1 x 56 name the 2-D multi-step wave strips (1 x 56 also the
-	// four-step field strips, where their body was chosen)
-	if (s->geom.dim == 2 && ty == 1 && (tz == kSteps8Cols || tz == kSteps4Cols))
-		opt = tz == kSteps8Cols ? 13 : s->tuned && s->tile.opt == 16 ? 16 : 14;
+	// 1 x 48 and 1 x 56 name the 2-D multi-step wave strips, 1 x 56 on a vector
+	// grid the four-step field strips
+	const bool vec = s->desc.vector != 0;
+	if (s->geom.dim == 2 && ty == 1 && (tz == kSteps8Cols || tz == kSteps4Cols)) {
+		opt = tz == kSteps8Cols ? 13 : vec ? 16 : 14;
+		if (!body_takes_grid(s, opt)) return fail(MMSPX_EINVAL, "no compiled tile of that shape for this grid");
+	}
 	// 3-D two-step bodies: 32 x 32 tiles run body 7 only; body 6 runs 32 x 64
 	if (s->geom.dim == 3 && ty == 32 && tz == 32) opt = 7;
 	else if (s->geom.dim == 3 && s->tuned && s->tile.opt == 6 && ty == 32 && tz == 64) opt = 6;
 	else if (s->geom.dim == 3 && s->tuned && (s->tile.opt == 8 || s->tile.opt == 12)) opt = s->tile.opt;
-	// 26 x 52, 16 x 16 and the tiles of 56 columns name the 3-D four-level march
-	if (s->geom.dim == 3 && ((s->tuned && s->tile.opt == 15 && march4_tile_known(s->desc.precision, ty, tz)) ||
-	                         (ty == 26 && tz == 52) || (ty == 16 && tz == 16) ||
-	                         (tz == 56 && march4_tile_known(s->desc.precision, ty, tz))))
+	// 26 x 52, 16 x 16 and the tiles of 56 columns name the 3-D four-level march,
+	// on a vector grid its tiles name the field march
+	if (s->geom.dim == 3 && !vec && ((s->tuned && s->tile.opt == 15 && march4_tile_known(s->desc.precision, ty, tz)) ||
+	                                 (ty == 26 && tz == 52) || (ty == 16 && tz == 16) ||
+	                                 (tz == 56 && march4_tile_known(s->desc.precision, ty, tz))))
 		opt = 15;
-	// the 3-D field march keeps its body on its own tiles
-	if (s->geom.dim == 3 && s->tuned && s->tile.opt == 17 &&
-	    fmarch_tile_known(s->desc.precision, s->geom.fields, ty, tz))
-		opt = 17;
+	if (s->geom.dim == 3 && vec && fmarch_tile_known(s->desc.precision, s->geom.fields, ty, tz)) opt = 17;
 	TuneChoice t{2, ty, tz, chunk, opt};
 	if (!tile_known(s->geom, t)) return fail(MMSPX_EINVAL, "no compiled tile of that shape for this grid");
 	s->tile = t;
@@ -516,6 +528,7 @@ int mmspx_set_tile_options(mmspx_state* s, int body)
 	     s->geom.dim != 2) ||
 	    (((body >= 6 && body <= 8) || body == 12 || body == 15 || body == 17) && s->geom.dim != 3))
 		return fail(MMSPX_EINVAL, "unknown tile body");
+	if (!body_takes_grid(s, body)) return fail(MMSPX_EINVAL, "this tile body does not run grids of this kind and field count");
 	if (!s->tuned) {
 		s->tile = one_step_choice(s->geom, s->desc.precision, MMSPX_CH_DW);
 		s->tuned = true;
@@ -534,6 +547,8 @@ int mmspx_set_tile_options(mmspx_state* s, int body)
 		} else if (body == 4 || body == 5) {
 			s->tile.ty = 1;
 			s->tile.tz = kWaveCols;
+		} else if (s->tile.ty == 1 && (s->tile.tz == kSteps8Cols || s->tile.tz == kSteps4Cols)) {
+			s->tile.tz = kWaveCols;  // the multi-step strips' columns are no other body's
 		}
 	}
 	// 3-D: keep a tile the body runs (32 x 32 tiles run body 7 only, body 6
@@ -566,8 +581,9 @@ int mmspx_set_tile_options(mmspx_state* s, int body)
 		} else if (body == 7) {
 			s->tile.ty = 32;
 			s->tile.tz = 32;
-		} else if (body == 6 || (s->tile.ty == 32 && s->tile.tz == 32)) {
-			s->tile.ty = 32;
+		} else if (body == 6 || (ty == 32 && tz == 32) || !tile_known(s->geom, TuneChoice{2, ty, tz, 2, 0})) {
+			// (the tiles of bodies 15 and 17 are not the others'; 8 x 64 is every vector model's)
+			s->tile.ty = s->desc.vector && body != 6 && !(ty == 32 && tz == 32) ? 8 : 32;
 			s->tile.tz = 64;
 		}
 	}
