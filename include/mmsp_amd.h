@@ -354,12 +354,21 @@ int mmspx_batch_autotune(mmspx_batch* b, int trial_steps, char* report, size_t r
  * columns by rows_per_item rows with blocks_per_cu persistent workgroups per
  * CU, or, for Allen-Cahn with cells > 0, runs of `cells` consecutive nodes.
  * strip_width 48 selects temporal blocks (periodic Allen-Cahn members only):
- * 16 x 48-node blocks taking rows_per_item (1..8) steps per pass over HBM. */
+ * 16 x 48-node blocks taking rows_per_item (1..8) steps per pass over HBM.
+ * blocks_per_cu 0 selects the multi-step kernels, the default where they take
+ * every member (Allen-Cahn and Cahn-Hilliard in the MMSPX_F64 and MMSPX_F32
+ * forms, axes periodic on both sides or on neither): strip_width 48 takes
+ * eight levels of the update per pass, 56 four, in strips of rows_per_item
+ * rows; 3-D members run the four-level march on a tile of the library's
+ * choice, whose columns are strip_width where all members are 3-D
+ * (rows_per_item then its planes). */
 int mmspx_batch_set_tile(mmspx_batch* b, int strip_width, int rows_per_item, int blocks_per_cu, int cells);
 /* Returns 1 when the tile came from the autotuner, 0 for the default. For
  * Allen-Cahn batches run by runs of consecutive nodes, strip_width and
  * blocks_per_cu are 0 and rows_per_item holds the nodes per workgroup; for
- * temporal blocks strip_width is 48 and rows_per_item the steps per pass. */
+ * temporal blocks strip_width is 48 and rows_per_item the steps per pass; for
+ * the multi-step kernels blocks_per_cu is 0. Except for runs of consecutive
+ * nodes, mmspx_batch_set_tile takes what this returns. */
 int mmspx_batch_get_tile(const mmspx_batch* b, int* strip_width, int* rows_per_item, int* blocks_per_cu);
 
 /* ---- serving: continuous batching of solves ------------------------------ */

@@ -498,7 +498,8 @@ class Batch:
     def set_tile(self, strip_width=256, rows_per_item=32, blocks_per_cu=8, cells=0):
         """Strips (width 64/128/256), runs of `cells` nodes (Allen-Cahn), or with
         strip_width 48 temporal blocks taking rows_per_item steps per pass
-        (periodic Allen-Cahn)."""
+        (periodic Allen-Cahn); with blocks_per_cu 0 the multi-step kernels, the
+        default, on strips of 48 or 56 columns (mmspx_batch_set_tile)."""
         check(lib.mmspx_batch_set_tile(self._h, strip_width, rows_per_item, blocks_per_cu, cells))
 
     def get_tile(self):

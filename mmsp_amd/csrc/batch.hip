@@ -543,6 +543,20 @@ void mmspx_batch_destroy(mmspx_batch* b)
 	staging_release();
 }
 
+static bool multi_step(const BatchTile& t) { return t.lv > 0 || t.y3 > 0; }
+
+// The default tile: the multi-step kernels where they take every member.
+static BatchTile default_tile(const mmspx_batch* b)
+{
+	// Cahn-Hilliard: 2-D members by wave strips (faster than the LDS row strips)
+	const bool ch = b->model == MMSPX_CH || b->model == MMSPX_CH_DW;
+	BatchTile t = ch ? BatchTile{kChWaveOut, 8, 16, 8, 0} : BatchTile{256, 32, 16, 8, 0};
+	std::vector<const Geom*> gs;
+	for (const Geom& g : b->geom) gs.push_back(&g);
+	batch_multi_step_choice(b->model, b->prec, gs.data(), b->count, &t);
+	return t;
+}
+
 int mmspx_batch_create(const mmspx_desc* descs, int count, int model, mmspx_batch** out)
 {
 	if (!out) return fail(MMSPX_EINVAL, "null output pointer");
@@ -584,13 +598,7 @@ int mmspx_batch_create(const mmspx_desc* descs, int count, int model, mmspx_batc
 	}
 	staging_retain();
 	b->params.assign(count, ModelParams{});
-	// Cahn-Hilliard: 2-D members by wave strips (faster than the LDS row strips)
-	if (model == MMSPX_CH || model == MMSPX_CH_DW) b->tile = BatchTile{kChWaveOut, 8, 16, 8, 0};
-	{
-		std::vector<const Geom*> gs;
-		for (const Geom& g : b->geom) gs.push_back(&g);
-		batch_multi_step_choice(model, b->prec, gs.data(), count, &b->tile);
-	}
+	b->tile = default_tile(b);
 	b->cus = device_cus();
 	b->arena_bytes = total;
 	const size_t red = (size_t)b->fields * 2 * kRedBlocks * sizeof(double);
@@ -708,6 +716,18 @@ static bool all_members_periodic(const mmspx_batch* b)
 int mmspx_batch_set_tile(mmspx_batch* b, int tz, int chunk, int blocks_per_cu, int cells)
 {
 	if (!b) return fail(MMSPX_EINVAL, "null batch");
+	if (blocks_per_cu == 0 && cells == 0) {  // the multi-step kernels
+		BatchTile t = default_tile(b);
+		const bool strips = t.lv > 0 && (tz == kSteps8Cols || tz == kSteps4Cols);
+		const bool march = t.lv == 0 && t.y3 > 0 && tz == t.z3;
+		if ((!strips && !march) || chunk < 1 || chunk > 4096)
+			return fail(MMSPX_EINVAL, "no workgroups per CU: the multi-step kernels, strips of 48 or 56 columns (3-D members "
+			                          "alone: the tile's columns), for members they take");
+		if (strips) t.lv = (64 - tz) / 2;
+		(strips ? t.chunk : t.chunk3) = chunk;
+		b->tile = t;
+		return upload_plan(b);
+	}
 	if (tz == kTbCols) {  // temporal blocks: chunk = steps per pass
 		if (b->model != MMSPX_AC || !all_members_periodic(b) || chunk < 1 || chunk > kTbMaxSteps || blocks_per_cu < 1)
 			return fail(MMSPX_EINVAL, "temporal blocks: periodic Allen-Cahn members, 1..8 steps per pass");
@@ -729,6 +749,12 @@ int mmspx_batch_get_tile(const mmspx_batch* b, int* tz, int* chunk, int* blocks_
 {
 	if (!b) return fail(MMSPX_EINVAL, "null batch");
 	const BatchTile& t = b->tile;
+	if (t.lv == 0 && t.y3 > 0) {
+		if (tz) *tz = t.z3;
+		if (chunk) *chunk = t.chunk3;
+		if (blocks_per_cu) *blocks_per_cu = 0;
+		return b->tuned ? 1 : 0;
+	}
 	if (tz) *tz = t.lv > 0 ? 64 - 2 * t.lv : t.tb > 0 ? kTbCols : t.cells > 0 ? 0 : t.tz;
 	if (chunk) *chunk = t.tb > 0 ? t.tb : t.cells > 0 ? t.cells : t.chunk;
 	if (blocks_per_cu) *blocks_per_cu = t.cells > 0 || t.lv > 0 ? 0 : t.bpc;
@@ -750,7 +776,8 @@ int mmspx_batch_autotune(mmspx_batch* b, int trial_steps, char* report, size_t r
 	const int64_t steps0 = b->steps_done, p2 = b->passes2, p3 = b->passes3;
 	const BatchTile keep = b->tile;
 	std::vector<BatchTile> cand;
-	if (b->tile.lv > 0 || b->tile.y3 > 0) cand.push_back(b->tile);  // the multi-step kernels as chosen
+	if (multi_step(keep)) cand.push_back(keep);
+	if (multi_step(default_tile(b))) cand.push_back(default_tile(b));  // also after another tile was set
 	for (int tz : {64, 128, 256})
 		for (int chunk : {16, 32, 64, 128})
 			for (int bpc : {4, 8, 16}) cand.push_back(BatchTile{tz, chunk, 16, bpc, 0});
@@ -783,7 +810,7 @@ int mmspx_batch_autotune(mmspx_batch* b, int trial_steps, char* report, size_t r
 		sec = sec / steps * trial_steps;
 		char line[160];
 		std::snprintf(line, sizeof line, "tz=%d chunk=%d blocks_per_cu=%d cells=%d steps_per_pass=%d us_per_step=%.2f\n",
-		              t.lv > 0 ? 64 - 2 * t.lv : t.tz, t.chunk, t.bpc, t.cells, spp > 1 ? spp : 0, sec / trial_steps * 1e6);
+		              t.lv > 0 ? 64 - 2 * t.lv : t.tz, t.chunk, multi_step(t) ? 0 : t.bpc, t.cells, spp > 1 ? spp : 0, sec / trial_steps * 1e6);
 		rep += line;
 		if (sec < best) {
 			best = sec;
