@@ -13,6 +13,10 @@
 // The server's transfers, which run beside its steps, were no faster this way
 // (22.0 and 22.8 ms for 16 requests) and stay with the runtime.
 //
+// Memory of the caller's that the runtime knows already (pinned, managed, of a
+// device) takes one direct copy: a pinned destination of 8 MiB 156 us, through
+// the area 337.
+//
 // The pinned memory is one area per process: at most 16 MiB, made when a
 // transfer first needs it, grown once, given back when the last state or
 // batch is destroyed. One transfer holds it at a time; another thread's transfer that
@@ -151,10 +155,19 @@ void staging_release()
 	give_back(g_staging);
 }
 
+// pageable: memory the runtime does not know
+static bool pageable(const void* p)
+{
+	hipPointerAttribute_t a;
+	if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type == hipMemoryTypeUnregistered;
+	(void)hipGetLastError();
+	return true;
+}
+
 int copy_to_host(void* dst, const void* src, size_t bytes, hipStream_t st)
 {
-	std::unique_lock<std::mutex> area(g_staging.busy, std::try_to_lock);
-	if (bytes > 0 && area.owns_lock() && ready(g_staging, bytes, bytes > kStagedDown, st)) {
+	std::unique_lock<std::mutex> area(g_staging.busy, std::defer_lock);
+	if (bytes > 0 && pageable(dst) && area.try_lock() && ready(g_staging, bytes, bytes > kStagedDown, st)) {
 		if (bytes > kStagedDown)
 			return download_pieces(g_staging, (char*)dst, (const char*)src, bytes, st,
 			                       bytes < ((size_t)16 << 20) ? 2 : bytes < ((size_t)48 << 20) ? 4 : 8);
@@ -172,7 +185,7 @@ int copy_to_host(void* dst, const void* src, size_t bytes, hipStream_t st)
 int copy_to_device(void* dst, const void* src, size_t bytes, hipStream_t st)
 {
 	std::unique_lock<std::mutex> area(g_staging.busy, std::defer_lock);
-	if (bytes > 0 && bytes <= kStagedUp && area.try_lock() && ready(g_staging, bytes, false, st)) {
+	if (bytes > 0 && bytes <= kStagedUp && pageable(src) && area.try_lock() && ready(g_staging, bytes, false, st)) {
 		// in pieces, so that the copy into pinned memory overlaps the transfer
 		constexpr size_t piece = kSlotBytes / 2;
 		hipError_t e = hipSuccess;
