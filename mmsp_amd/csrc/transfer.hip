@@ -19,8 +19,13 @@
 //
 // The pinned memory is one area per process: at most 16 MiB, made when a
 // transfer first needs it, grown once, given back when the last state or
-// batch is destroyed. One transfer holds it at a time; another thread's transfer that
-// finds it taken uses hipMemcpyAsync as before.
+// batch is destroyed. Making it and giving it back takes 20 us (2 MiB) to 75, more
+// than one small transfer saves, and a program that makes a state for each solve
+// would pay it each time (create, upload, ten steps, download, destroy: 128^2
+// 153 us plain, 171 to 186 with the area; 700^2 555 and 630; 1024^2 925 and 900,
+// 128^3 1690 and 1470): downloads of 8 MiB and more make it at once, smaller
+// transfers when eight of them have asked for it. One transfer holds it at a
+// time; another thread's transfer that finds it taken uses hipMemcpyAsync.
 #include <algorithm>
 #include <cstring>
 #include <mutex>
@@ -34,6 +39,8 @@ namespace {
 
 constexpr size_t kSlotBytes = (size_t)1 << 20;
 constexpr int kSlots = 16;
+constexpr size_t kAtOnce = 8 * kSlotBytes;
+constexpr int kAsk = 8;
 constexpr size_t kStagedDown = 2 * kSlotBytes, kStagedUp = kSlotBytes + kSlotBytes / 2;
 
 struct Staging {
@@ -42,6 +49,7 @@ struct Staging {
 	int users = 0;
 	char* base = nullptr;
 	size_t bytes = 0;
+	int asked = 0;       // transfers that found no area of their size
 	int device = -1;
 	hipEvent_t ev[kSlots] = {};
 };
@@ -57,6 +65,7 @@ void give_back(Staging& s)
 	if (s.base) (void)hipHostFree(s.base);
 	s.base = nullptr;
 	s.bytes = 0;
+	s.asked = 0;
 	s.device = -1;
 }
 
@@ -72,6 +81,7 @@ bool ready(Staging& s, size_t need, bool events, hipStream_t st)
 	}
 	const size_t want = need <= 2 * kSlotBytes ? 2 * kSlotBytes : kSlots * kSlotBytes;
 	if (s.bytes < want) {
+		if (need < kAtOnce && ++s.asked <= kAsk) return false;
 		// relaxed: another thread's stream capture is not ours to disturb
 		hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
 		(void)hipThreadExchangeStreamCaptureMode(&mode);
@@ -86,6 +96,7 @@ bool ready(Staging& s, size_t need, bool events, hipStream_t st)
 			return false;
 		}
 		s.bytes = want;
+		s.asked = 0;
 		s.device = dev;
 	}
 	for (int k = 0; events && k < kSlots; k++)
