@@ -457,7 +457,8 @@ TuneChoice default_choice(const Geom& g, int prec, int model)
 // - one or two steps of 2-D grain growth and Zener pinning: the split strips
 //   (512^2 x 32 FP32 one 21.2 and 16.4, two 29.3 and 22.9).
 // - one step of 3-D Allen-Cahn: the plane march (FP64 64^3 10.2 and 5.8, 256^3
-//   69 and 45; FP32 41 and 24); two, from 2^20 nodes: that march two steps per
+//   69 and 45; FP32 41 and 24), in FP32 up to 2^20 nodes on 16 x 32 tiles (64^3 5.8
+//   against 7.0 on that march's own default, 64 x 128 x 128 6.4 against 7.4); two, from 2^20 nodes: that march two steps per
 //   pass where it fits (256^3 FP64 73 and 60, FP32 42 and 35).
 // - one step of 3-D Cahn-Hilliard: march4_last_step_choice.
 // - one step of 3-D grain growth and Zener pinning: the plane march (192^3 x 8
@@ -482,7 +483,7 @@ TuneChoice pass_choice(const Geom& g, int prec, int model, const TuneChoice& ful
 		break;
 	case 15:
 		if (model == MMSPX_AC) {
-			if (left == 1) t = one_step_choice(g, prec, model);
+			if (left == 1) t = prec == MMSPX_F32 && nodes <= ((int64_t)1 << 20) ? TuneChoice{2, 16, 32, 4, 8} : one_step_choice(g, prec, model);
 			else if (left == 2 && nodes >= ((int64_t)1 << 20) && !march2_choice(g, prec, model, &t)) t = full;
 		} else if (!march4_last_step_choice(g, prec, full, &t)) {
 			t = full;

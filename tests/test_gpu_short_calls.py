@@ -66,6 +66,17 @@ def check(model, shape, q, bc, bodies, prec):
             assert np.array_equal(g.download(), expected(model, a, steps, prec, bc)), steps
 
 
+def test_one_step_of_small_single_precision_marches():
+    a = start((24, 33, 40), 1, 3650, "f32")
+    with mx.Grid(a.shape, precision="f32") as g:
+        g.upload(a)
+        g.step("ac", PARAMS["ac"], 5)  # a pass of four and one step
+        g.step("ac", PARAMS["ac"], 1)
+        k = g.get_kernel()
+        assert (k["ty"], k["tz"], k["chunk"], k["opt"]) == (16, 32, 4, 8)
+        assert np.array_equal(g.download(), expected("ac", a, 6, "f32", None))
+
+
 # large grids: two steps of 3-D Allen-Cahn, one of 3-D Cahn-Hilliard, two of
 # Allen-Cahn between walls; 2-D Allen-Cahn too large for the temporal blocks
 @pytest.mark.parametrize("model,shape,bc,prec,steps,bodies", [
