@@ -150,9 +150,6 @@ __device__ __forceinline__ void fmarch(const typename Form<PREC>::S* __restrict_
 			}
 			const typename F::L lap = (tx + ty) + tz;
 			value(k, F::gg(y, tot[s][r0 + k][lane], lap, p));
-#ifdef SBK
-			if (k % SBK == SBK - 1) __builtin_amdgcn_sched_barrier(0);
-#endif
 		}
 	};
 	// the iteration at plane P = xb - H + i; j = i mod 3 is known at compile
@@ -187,16 +184,7 @@ __device__ __forceinline__ void fmarch(const typename Form<PREC>::S* __restrict_
 	load(f[0]);
 	load(f[1]);
 	load(f[2]);
-	// the ring row of the first centre plane
-	S ring1 = 0;
-	{
-		const int x1 = wrap(xb - L + 1, nx);
-		if (first || last) ring1 = load_at(af + (int64_t)x1 * plane + rrow, zc);
-		const S keep = rgc;
-		rgc = ring1;
-		exchange(f[1], 0);
-		rgc = keep;
-	}
+	exchange(f[1], 0);  // rgc is the ring row of the first centre plane, xb - L + 1
 	const int n = xe - xb + H + LEVELS - 1;
 #pragma unroll
 	for (int i = 0; i < 2 * H; i++) iter(i, i % 3, 1 + i / 2);
