@@ -454,12 +454,16 @@ TuneChoice default_choice(const Geom& g, int prec, int model)
 //   two steps 19.5 and 17.1; two at 700^2 7.1 and 8.6, at 4096^2 42 and 45).
 // - one step of 2-D Cahn-Hilliard: its wave strips (1024^2 FP64 8.4 and 6.5,
 //   FP32 7.3 and 5.7; 2048^2 FP32 14.6 and 10.1).
-// - one or two steps of 2-D grain growth and Zener pinning: the split strips
-//   (512^2 x 32 FP32 one 21.2 and 16.4, two 29.3 and 22.9).
-// - one step of 3-D Allen-Cahn: the plane march (FP64 64^3 10.2 and 5.8, 256^3
-//   69 and 45; FP32 41 and 24), in FP32 up to 2^20 nodes on 16 x 32 tiles (64^3 5.8
-//   against 7.0 on that march's own default, 64 x 128 x 128 6.4 against 7.4); two, from 2^20 nodes: that march two steps per
-//   pass where it fits (256^3 FP64 73 and 60, FP32 42 and 35).
+// - one or two steps of 2-D grain growth and Zener pinning from 2^21 values (nodes
+//   x fields): the split strips (512^2 x 32 FP32 one 21.2 and 16.4, two 29.3 and
+//   22.9). Below, their rows a wave are a longer serial march than the cut pass
+//   (at the end of a call of 48 steps: 64^2 x 32 FP32 one 6.2 and 12.8 us, 309 x
+//   73 x 2 FP64 3.5 and 7.1).
+// - one step of 3-D Allen-Cahn from 2^18 nodes: the plane march (FP64 256^3 69 and
+//   45; FP32 41 and 24; below, after 48 steps, 48^3 FP64 4.8 and 5.8), in FP32 up
+//   to 2^20 nodes on 16 x 32 tiles (64^3 5.8 against 7.0 on that march's own
+//   default, 64 x 128 x 128 6.4 against 7.4); two, from 2^20 nodes: that march two
+//   steps per pass where it fits (256^3 FP64 73 and 60, FP32 42 and 35).
 // - one step of 3-D Cahn-Hilliard: march4_last_step_choice.
 // - one step of 3-D grain growth and Zener pinning: the plane march (192^3 x 8
 //   FP32 157 and 120, 256^3 x 8 392 and 243, 96^3 x 4 16.4 and 11.9), but for 8
@@ -483,14 +487,15 @@ TuneChoice pass_choice(const Geom& g, int prec, int model, const TuneChoice& ful
 		break;
 	case 15:
 		if (model == MMSPX_AC) {
-			if (left == 1) t = prec == MMSPX_F32 && nodes <= ((int64_t)1 << 20) ? TuneChoice{2, 16, 32, 4, 8} : one_step_choice(g, prec, model);
+			if (left == 1 && nodes >= ((int64_t)1 << 18))
+				t = prec == MMSPX_F32 && nodes <= ((int64_t)1 << 20) ? TuneChoice{2, 16, 32, 4, 8} : one_step_choice(g, prec, model);
 			else if (left == 2 && nodes >= ((int64_t)1 << 20) && !march2_choice(g, prec, model, &t)) t = full;
 		} else if (!march4_last_step_choice(g, prec, full, &t)) {
 			t = full;
 		}
 		break;
 	case 16:
-		if (left <= 2) t = one_step_choice(g, prec, model);
+		if (left <= 2 && nodes * g.fields >= ((int64_t)1 << 21)) t = one_step_choice(g, prec, model);
 		break;
 	case 17: {
 		const int pad = (g.n[2] + 63) / 64 * 64 - g.n[2];

@@ -20,9 +20,11 @@ CASES = [
     ("ac", (40, 60), 1, WALLS, {1: (2,), 2: (13, 14), 5: (13, 14), 9: (13, 14)}),
     ("ch", (40, 60), 1, WALLS, {1: (0,), 2: (13, 14), 3: (13, 14), 5: (13, 14)}),
     ("ch_dw", (40, 60), 1, None, {1: (0,), 2: (13, 14), 3: (13, 14), 5: (13, 14)}),
-    ("gg", (40, 60), 4, None, {1: (11,), 2: (11,), 3: (16,), 5: (16,), 6: (16,)}),
-    ("zener", (40, 60), 16, None, {1: (10,), 2: (10,), 3: (16,), 6: (16,)}),
-    ("ac", (20, 30, 40), 1, None, {1: (8,), 2: (15,), 3: (15,), 5: (15,), 6: (15,)}),
+    ("gg", (40, 60), 4, None, {1: (16,), 2: (16,), 3: (16,), 5: (16,), 6: (16,)}),
+    ("gg", (270, 250), 32, None, {1: (10,), 2: (10,), 3: (16,), 5: (16,), 6: (16,)}),
+    ("zener", (350, 380), 16, None, {1: (10,), 2: (10,), 3: (16,), 6: (16,)}),
+    ("ac", (20, 30, 40), 1, None, {1: (15,), 2: (15,), 5: (15,)}),
+    ("ac", (62, 66, 66), 1, None, {1: (8,), 2: (15,), 3: (15,), 5: (15,), 6: (15,)}),
     ("ch", (20, 30, 40), 1, None, {1: (15,), 2: (15,), 3: (15,)}),
 ]
 # 3-D grain growth: the field march by precision; in FP64 its single step too,
@@ -67,7 +69,7 @@ def check(model, shape, q, bc, bodies, prec):
 
 
 def test_one_step_of_small_single_precision_marches():
-    a = start((24, 33, 40), 1, 3650, "f32")
+    a = start((62, 66, 66), 1, 3650, "f32")
     with mx.Grid(a.shape, precision="f32") as g:
         g.upload(a)
         g.step("ac", PARAMS["ac"], 5)  # a pass of four and one step
