@@ -328,9 +328,9 @@ int mmspx_copy_bandwidth(size_t bytes, int reps, double* bytes_per_s);
 
 /* ---- batches: many independent grids advanced together ---------------------
  * All members share model, precision and field count and advance by the same
- * number of steps; extents and parameters may differ. One persistent kernel
- * launch per step walks a device work list holding every member's tiles
- * (2-D Allen-Cahn / grain growth, periodic 2-D and 3-D Cahn-Hilliard; 3-D
+ * number of steps; extents and parameters may differ. One kernel launch per
+ * pass (one step, or several on the multi-step kernels and temporal blocks)
+ * walks a device work list holding every member's tiles (2-D Allen-Cahn / grain growth, periodic 2-D and 3-D Cahn-Hilliard; 3-D
  * members take a second launch); multi-step runs replay a captured hipGraph.
  * No counterpart in the reference, which advances one grid per process. */
 typedef struct mmspx_batch mmspx_batch;

@@ -153,7 +153,7 @@ int launch_fused_step(const Geom& g, int prec, const ModelParams& p, const void*
 bool fused_needs_plane(const Geom& g, int model, const TuneChoice& t);
 int fused_steps_per_launch(int model, const TuneChoice& t);
 TuneChoice default_choice(const Geom& g, int prec, int model);
-// the default without the 2-D multi-step wave strips and the four-level march
+// the default without the multi-step kernels
 TuneChoice one_step_choice(const Geom& g, int prec, int model);
 // the kernel of a call's next pass where `left` steps remain and the call runs
 // the default `full`

@@ -18,9 +18,10 @@
 // operands in the same order (KIND 3 holds field 0, zener.cpp:117-135), so a
 // pass gives the bits of single steps.
 //
-// Bound by memory and the exchange together: 256^3 x 8 FP32 in three-step
-// passes of 500 us moves 1.9 TB/s of compulsory bytes (3.6 with the halo it
-// reads) while LDS and vector work each take about 40 % of the time. R and L
+// Bound by the exchange and vector work together: 256^3 x 8 FP32 in three-step
+// passes of 500 us moves 2.4 TB/s, vector work (2.4e8 instructions a launch) is
+// about 46 % of the time at 2.4 cycles each, and the waves wait 38 % of theirs at
+// the two barriers; no bank conflicts. R and L
 // are what 128 registers a lane hold (6 to 12 values a row). Stores go under
 // one condition a row and all addresses are a scalar row start plus one lane
 // offset: left to itself the compiler kept a 64-bit address per row in vector

@@ -506,8 +506,11 @@ TuneChoice pass_choice(const Geom& g, int prec, int model, const TuneChoice& ful
 	return t.variant == 2 ? t : full;
 }
 
-// Defaults come from sweeps of the candidates below on MI355X (the figures
-// quoted are microseconds per step from those sweeps).
+// The defaults where no multi-step kernel runs (the reference's float form, noise,
+// other boundaries, other field counts, Ostwald ripening, multi-phase grain
+// growth) and, by pass_choice, of a call's last steps. From sweeps of the
+// candidates below on MI355X (the figures quoted are microseconds per step from
+// those sweeps).
 TuneChoice one_step_choice(const Geom& g, int prec, int model)
 {
 	if (!fused_supported(g, prec, model)) return TuneChoice{1, 0, 0, 0, 0};
@@ -573,7 +576,8 @@ TuneChoice one_step_choice(const Geom& g, int prec, int model)
 		while (chunk > 4 && tiles * ((g.n[0] + chunk - 1) / chunk) < 512) chunk /= 2;
 		return TuneChoice{2, ty, tz, chunk, 8};
 	}
-	// Allen-Cahn: periodic grids take temporal blocks of 48 columns and 8
+	// Allen-Cahn, in the reference's float form and for the last steps of a call
+	// (pass_choice): periodic grids take temporal blocks of 48 columns and 8
 	// steps per pass (512^2: 2.05 us per step in FP64 against 4.58 us for one
 	// thread per node). Block heights from a sweep of 8, 16, 32 rows (on 512,
 	// 1024, 1024 threads) x 4, 8 steps, sides 256 to 4096: 16 rows up to 2^16

@@ -15,11 +15,12 @@
 // Cahn-Hilliard 42 us per step: 22 and 20). Here vector work is 73 % of the
 // time at the rates the instructions reach (4.3 cycles for a double add or a
 // shift), the rest waits at the barrier; 16 waves of two rows, the most a
-// workgroup holds, or 12 of four where the grid gives each enough planes (320^3
-// 67 against 84 us): 256^3 FP64 Cahn-Hilliard 35.7 us per step, Allen-Cahn 24.4
-// (8 waves of four rows 38.3 and 25.6; a column pair per lane, which halves
-// the shifts, 40.1 and 26.4; levels two planes apart instead of one, so that
-// none waits for another, 37.3 and 25.4).
+// workgroup holds, or 12 of four where the grid gives each enough planes. Whole
+// calls at 256^3 FP64, us per step: Cahn-Hilliard 38.0, Allen-Cahn 25.1 where
+// every coefficient is one and 27.1 otherwise; 320^3 Cahn-Hilliard 70.6. Tried
+// at 256^3 in a loop of their own, Cahn-Hilliard and Allen-Cahn: 8 waves of four
+// rows 7 and 5 % slower, a column pair per lane (half the shifts) 12 and 8 %,
+// levels two planes apart, so that none waits for another, 4 %.
 #pragma once
 
 #include "march4.hpp"
