@@ -302,8 +302,9 @@ int mmspx_set_tile_options(mmspx_state* s, int body);
  * 3: temporal blocks, or 3-D register queues on 1024 threads; 4 and 5: the
  * split strips on two and four waves; 13 and 14: the multi-step wave strips; 15: the
  * 3-D four-level march; 16: the four-step field strips; 17: the 3-D field
- * march). Before any tile is
- * set, reports what the last step ran (the Cahn-Hilliard default before any step). */
+ * march). Before any tile is set, reports what the last step's first pass ran
+ * (the Cahn-Hilliard default before any step), a default on body 15 or 17 as
+ * the body of the pass it stands for; mmspx_get_kernel names its own. */
 int mmspx_get_tile(const mmspx_state* s, int* ty, int* tz, int* chunk);
 /* The same numbers for the kernel that the last mmspx_step ran its first pass
  * on (before any step: the tile set, or the Cahn-Hilliard default), with that
@@ -330,8 +331,8 @@ int mmspx_copy_bandwidth(size_t bytes, int reps, double* bytes_per_s);
  * All members share model, precision and field count and advance by the same
  * number of steps; extents and parameters may differ. One kernel launch per
  * pass (one step, or several on the multi-step kernels and temporal blocks)
- * walks a device work list holding every member's tiles (2-D Allen-Cahn / grain growth, periodic 2-D and 3-D Cahn-Hilliard; 3-D
- * members take a second launch); multi-step runs replay a captured hipGraph.
+ * walks a device work list holding every member's tiles (2-D Allen-Cahn / grain
+ * growth, periodic 2-D and 3-D Cahn-Hilliard; 3-D members take a second launch); multi-step runs replay a captured hipGraph.
  * No counterpart in the reference, which advances one grid per process. */
 typedef struct mmspx_batch mmspx_batch;
 
