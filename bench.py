@@ -249,6 +249,7 @@ def bench_batch_ac(args):
             r64 = g.download()
         err = max(err, float(np.abs(out32[m] - r64).max() / np.abs(r64).max()))
     value = cells * K / dev_s
+    kernel = "ac_batch" if tile["blocks_per_cu"] else "steps2d_batch"
     return {
         "metric": "cell-updates/s",
         "value": value,
@@ -281,8 +282,8 @@ def bench_batch_ac(args):
             "peak": HBM_PEAK_GBS,
             "unit": "GB/s",
             "frac": value * 8 / 1e9 / HBM_PEAK_GBS,
-            "traffic": traffic_from_profiles("ac_batch_batch_ac", tile),
-            "kernel": "ac_batch",
+            "traffic": traffic_from_profiles(kernel + "_batch_ac", tile),
+            "kernel": kernel,
             "algorithmic_bytes_per_launch": 8 * cells,
         },
     }
@@ -762,7 +763,7 @@ def main():
     elif tile["opt"] == 16:
         kname = "fields2d"
     elif tile["opt"] == 2:
-        kname = "wave_strips"
+        kname = "gga2d" if base == "gga" else "wave_strips"
     elif tile["opt"] in (4, 5):
         kname = "wave_strips_split"
     elif tile["opt"] in (9, 10, 11):

@@ -1,0 +1,12 @@
+// kernels_fused_ac_f64.hip -- the tiled kernels of Allen-Cahn and model A, FP64 form.
+#include "fused_launch.hpp"
+
+namespace mmspx {
+
+int launch_fused_ac_f64(MMSPX_FUSED_ARGS)
+{
+	(void)prec;
+	return launch_fused_ac<MMSPX_F64>(g, p, a, b, st, t, nsteps, aux);
+}
+
+}  // namespace mmspx

@@ -9,7 +9,7 @@
 // Hilliard runs its two passes (mu, then the update) exactly as the reference
 // does, so non-periodic boundaries see mu through the same mapping.
 //
-// The fused/tiled kernels (kernels_fused.hip) take over the hot shapes; these
+// The fused/tiled kernels (fused_launch.hpp) take over the hot shapes; these
 // serve every other case and are the in-library baseline the tuner compares
 // against.
 #include "device.hpp"

@@ -1,5 +1,5 @@
 // tiles.hpp -- per-tile device bodies shared by the single-grid kernels
-// (kernels_fused.hip) and the batched/persistent kernels (batch.hip).
+// (fused_launch.hpp) and the batched/persistent kernels (batch.hip).
 //
 // Every body reproduces the operation order of the generic kernels (and so of
 // the reference), so a grid gives the same bits whichever kernel advances it.
